@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "gsq_common.h"
 
@@ -454,21 +455,313 @@ __global__ void __launch_bounds__(1024) gdn_rec_seq_kernel(GdnArgs a) {
   }
 }
 
-hipError_t launch_gdn_seq(int dt, const GdnArgs& a, hipStream_t s) {
-  const int conv_dim = 2 * a.Hk * a.dk + a.Hv * a.dv;
-  const dim3 cgrid((unsigned)((conv_dim + 255) / 256), (unsigned)a.S, (unsigned)a.B), rgrid((unsigned)a.Hv, (unsigned)a.B);
-  const dim3 rblock((unsigned)(kGdnRowGroups * a.dv));
-  if (dt == MD_F16) {
-    hipLaunchKernelGGL(gdn_conv_seq_kernel<MD_F16>, cgrid, dim3(256), 0, s, a);
-    hipLaunchKernelGGL(gdn_rec_seq_kernel<MD_F16>, rgrid, rblock, 0, s, a);
-  } else if (dt == MD_BF16) {
-    hipLaunchKernelGGL(gdn_conv_seq_kernel<MD_BF16>, cgrid, dim3(256), 0, s, a);
-    hipLaunchKernelGGL(gdn_rec_seq_kernel<MD_BF16>, rgrid, rblock, 0, s, a);
-  } else {
-    hipLaunchKernelGGL(gdn_conv_seq_kernel<MD_F32>, cgrid, dim3(256), 0, s, a);
-    hipLaunchKernelGGL(gdn_rec_seq_kernel<MD_F32>, rgrid, rblock, 0, s, a);
+// The three kernels below run the sequence for key head dims 32, 64 and 128. The columns of a
+// head's state evolve independently given q, k, v, the decay and beta of each token; only the
+// output's RMSNorm couples them. So the serial part is split over columns (gdn_cols_seq_kernel:
+// no barrier and no exchange between waves inside a token), and what does not depend on the state
+// runs before it (gdn_prep_seq_kernel: convolution, q / k normalization) and after it
+// (gdn_out_seq_kernel: gated RMSNorm), in parallel over all tokens. Measured at 512 tokens, 48
+// heads of 128 x 128: gdn_rec_seq_kernel, which keeps a whole head in one workgroup and passes
+// seven barriers a token, 3017 us (5.9 us a token) after 28 us of convolution; these three 18 +
+// 161 + 11 us.
+
+constexpr int kGdnPrepTokens = 8;  // tokens per wave of gdn_prep_seq_kernel
+
+// Convolution + SiLU of 128 channels (2 per lane) over kGdnPrepTokens tokens, the window sliding in
+// registers; q and k channels are then RMS-normalized over their head (dk / 2 lanes, a power of
+// two) and scaled, so that `work` holds [q | k | v] rows ready for the recurrence. Bound by
+// memory: each input is read once per run of tokens (plus the window before it), each result
+// written once.
+template <int DT>
+__global__ void __launch_bounds__(256) gdn_prep_seq_kernel(GdnArgs a, bool pair) {
+  using E = Elem<DT>;
+  using T = typename E::T;
+  const int key_dim = a.Hk * a.dk, conv_dim = 2 * key_dim + a.Hv * a.dv, K = a.K, S = a.S;
+  const int lane = threadIdx.x & 63, wave = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int bb = blockIdx.z, t0 = blockIdx.y * kGdnPrepTokens;
+  const int cc = wave * 128 + 2 * lane, c = min(cc, conv_dim - 2);  // conv_dim is even
+  const bool on = cc < conv_dim;
+  const T* cst = static_cast<const T*>(a.conv) + (int64_t)bb * (K - 1) * conv_dim + c;
+  const T* q = static_cast<const T*>(a.qkv) + (int64_t)bb * S * a.qkv_stride + c;
+  // two neighbouring values: one load when every row's pairs are aligned to it
+  auto ld2 = [&](const T* p, float& x, float& y) {
+    if (pair) {
+      const struct alignas(2 * sizeof(T)) P { T e[2]; } v = *reinterpret_cast<const P*>(p);
+      x = E::ld(&v.e[0]);
+      y = E::ld(&v.e[1]);
+    } else {
+      x = E::ld(p);
+      y = E::ld(p + 1);
+    }
+  };
+  // window and weights right-aligned: slot kGdnMaxK - 1 is the current token
+  float w0[kGdnMaxK], w1[kGdnMaxK], in0[kGdnMaxK], in1[kGdnMaxK];
+  const T* cw = static_cast<const T*>(a.conv_w) + (int64_t)c * K;
+#pragma unroll
+  for (int i = 0; i < kGdnMaxK; ++i) {
+    const int j = i - (kGdnMaxK - K);  // window position, oldest 0
+    w0[i] = w1[i] = in0[i] = in1[i] = 0.f;
+    if (j >= 0) {
+      w0[i] = E::ld(cw + j);
+      w1[i] = E::ld(cw + K + j);
+      const int u = t0 - K + j;  // the window of token t0 - 1
+      if (u >= 0) {
+        ld2(q + (int64_t)u * a.qkv_stride, in0[i], in1[i]);
+      } else if (u >= -(K - 1)) {  // from the state
+        in0[i] = E::ld(cst + (int64_t)(K - 1 + u) * conv_dim);
+        in1[i] = E::ld(cst + (int64_t)(K - 1 + u) * conv_dim + 1);
+      }
+    }
   }
+  const float sc = c < key_dim ? 1.f / (float)a.dk : 1.f / sqrtf((float)a.dk);
+  const int half = a.dk >> 1;
+#pragma unroll
+  for (int i = 0; i < kGdnPrepTokens; ++i) {
+    const int t = t0 + i;
+    if (t >= S) break;
+#pragma unroll
+    for (int s = 0; s + 1 < kGdnMaxK; ++s) {
+      in0[s] = in0[s + 1];
+      in1[s] = in1[s + 1];
+    }
+    ld2(q + (int64_t)t * a.qkv_stride, in0[kGdnMaxK - 1], in1[kGdnMaxK - 1]);
+    float x = 0.f, y = 0.f;
+#pragma unroll
+    for (int s = 0; s < kGdnMaxK; ++s)
+      if (s >= kGdnMaxK - K) {
+        x += in0[s] * w0[s];
+        y += in1[s] * w1[s];
+      }
+    x = silu_f(x);
+    y = silu_f(y);
+    float ss = x * x + y * y;
+    for (int o = 1; o < half; o <<= 1) ss += __shfl_xor(ss, o, 64);
+    if (c < 2 * key_dim) {
+      const float rn = 1.f / sqrtf(ss / (float)a.dk + 1e-6f);
+      x = x * rn * sc;
+      y = y * rn * sc;
+    }
+    if (on) *reinterpret_cast<float2*>(a.work + ((int64_t)bb * S + t) * conv_dim + c) = make_float2(x, y);
+  }
+}
+
+constexpr int kGdnChunk = 16;  // tokens staged in LDS at a time
+constexpr int kGdnCols = 32;   // state columns per workgroup (8 per wave)
+
+// sum over the 8 lanes 8n .. 8n + 7
+__device__ __forceinline__ float sum8(float v) {
+  auto dpp = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                                 0xF, 0xF, false));
+  };
+  v += dpp(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  v += dpp(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  v += dpp(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
+  return v;
+}
+
+// The recurrence of kGdnCols columns of value head h: lane 8c + r of a wave holds rows 4r + 32i ..
+// + 3 (i < NR) of its column c in registers from the first token to the last, so a token is two
+// dot products over the column (in-lane sums, then three DPP steps over 8 lanes) and the update
+// between them: S = decay S; kv = S^T k; S += k beta (v - kv); o = S^T q. What bounds it is that
+// serial chain (one wave per SIMD at 48 heads of 128 columns: ~100 VALU instructions a token);
+// fewer lanes a column make it longer, more leave each lane too few rows to cover the reduction.
+// q, k, v of kGdnChunk tokens come by DMA into LDS one chunk ahead; the decay and beta of a chunk
+// are formed by its first lanes and broadcast by token; outputs replace v in `work` a chunk late.
+template <int DT, int NR>
+__global__ void __launch_bounds__(256) gdn_cols_seq_kernel(GdnArgs a) {
+  using E = Elem<DT>;
+  using T = typename E::T;
+  constexpr int CT = kGdnChunk, DK = 32 * NR, GT = DK / 2;  // GT: 16-byte granules of a token's q and k
+  __shared__ __attribute__((aligned(16))) float qk[2][CT * 2 * DK], vs[2][CT * kGdnCols], os[2][CT * kGdnCols];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int Hk = a.Hk, Hv = a.Hv, dv = a.dv, S = a.S, K = a.K, ns = dv / kGdnCols;
+  // key head fastest: the workgroups that read one key head's q and k are a multiple of Hk apart
+  // (one XCD when Hk is a multiple of 8)
+  const int kh = blockIdx.x % Hk, rest = blockIdx.x / Hk, slice = rest % ns, h = rest / ns * Hk + kh;
+  const int bb = blockIdx.y;
+  const int key_dim = Hk * DK, conv_dim = 2 * key_dim + Hv * dv, vch = 2 * key_dim + h * dv + slice * kGdnCols;
+  float* const work = a.work + (int64_t)bb * S * conv_dim;
+  const int r = lane & 7, col = wave * 8 + (lane >> 3);
+  float* const Sp = a.rec + (((int64_t)bb * Hv + h) * DK + 4 * r) * dv + slice * kGdnCols + col;
+  float st[4 * NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) st[4 * i + e] = Sp[(int64_t)(32 * i + e) * dv];
+  const float dtb = a.dt_bias[h], sa = a.ssm_a[h];
+
+  auto issue = [&](int t0, int buf) {  // tokens past the last one repeat it (not used)
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int e = (wave * NR + i) * 64 + lane, t = min(t0 + e / GT, S - 1), g = e % GT;
+      const float* src = work + (int64_t)t * conv_dim + (g < GT / 2 ? 0 : key_dim) + kh * DK + 4 * (g % (GT / 2));
+      __builtin_amdgcn_global_load_lds(src, (lds_ptr_t)(&qk[buf][(wave * NR + i) * 256]), 16, 0, 0);
+    }
+    if (wave < 2) {
+      const int e = wave * 64 + lane, t = min(t0 + e / 8, S - 1);
+      __builtin_amdgcn_global_load_lds(work + (int64_t)t * conv_dim + vch + 4 * (e % 8),
+                                       (lds_ptr_t)(&vs[buf][wave * 256]), 16, 0, 0);
+    }
+  };
+  auto load_ab = [&](int t0, float& av, float& bv) {  // lane t: token t0 + t
+    const T* abr = static_cast<const T*>(a.ab) + ((int64_t)bb * S + min(t0 + (lane & (CT - 1)), S - 1)) * a.ab_stride;
+    av = E::ld(abr + h);
+    bv = E::ld(abr + Hv + h);
+  };
+  auto store_o = [&](int t0, int buf) {
+    const int t = tid >> 4, c = 2 * (tid & 15);
+    if (t0 + t < S)
+      *reinterpret_cast<float2*>(work + (int64_t)(t0 + t) * conv_dim + vch + c) =
+          *reinterpret_cast<const float2*>(&os[buf][t * kGdnCols + c]);
+  };
+
+  float av, bv;
+  issue(0, 0);
+  load_ab(0, av, bv);
+  int buf = 0;
+  for (int t0 = 0; t0 < S; t0 += CT, buf ^= 1) {
+    // this chunk has landed; every wave is done with the other buffers
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    av += dtb;
+    const float sp = av > 20.f ? av : log1pf(expf(av));  // softplus (torch's threshold 20)
+    const int beta = __builtin_bit_cast(int, 1.f / (1.f + expf(-bv))), decay = __builtin_bit_cast(int, expf(sa * sp));
+    if (t0 + CT < S) {
+      issue(t0 + CT, buf ^ 1);
+      load_ab(t0 + CT, av, bv);
+    }
+    if (t0) store_o(t0 - CT, buf ^ 1);
+    const float* qb = &qk[buf][4 * r];
+    const float* vb = &vs[buf][col];
+    struct Tok { float4 q[NR], k[NR]; float v; };
+    auto fetch = [&](int t, Tok& x) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        x.q[i] = *reinterpret_cast<const float4*>(qb + t * 2 * DK + 32 * i);
+        x.k[i] = *reinterpret_cast<const float4*>(qb + t * 2 * DK + DK + 32 * i);
+      }
+      x.v = vb[t * kGdnCols];
+    };
+    // token t from x, while the next token's values (in bounds also past the chunk's last) go to nx
+    auto token = [&](int t, const Tok& x, Tok& nx) {
+      fetch(min(t + 1, CT - 1), nx);
+      const float d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(decay, t));
+      const float b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(beta, t));
+      float p[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const float kk[4] = {x.k[i].x, x.k[i].y, x.k[i].z, x.k[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          st[4 * i + e] *= d;
+          p[e] += st[4 * i + e] * kk[e];
+        }
+      }
+      const float delta = (x.v - sum8((p[0] + p[1]) + (p[2] + p[3]))) * b;
+      float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const float kk[4] = {x.k[i].x, x.k[i].y, x.k[i].z, x.k[i].w};
+        const float qq[4] = {x.q[i].x, x.q[i].y, x.q[i].z, x.q[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          st[4 * i + e] += kk[e] * delta;
+          o[e] += st[4 * i + e] * qq[e];
+        }
+      }
+      const float os_ = sum8((o[0] + o[1]) + (o[2] + o[3]));
+      if (r == 0) os[buf][t * kGdnCols + col] = os_;
+    };
+    Tok x0, x1;
+    fetch(0, x0);
+    const int n = min(CT, S - t0);
+    int t = 0;
+    for (; t + 1 < n; t += 2) {
+      token(t, x0, x1);
+      token(t + 1, x1, x0);
+    }
+    if (t < n) token(t, x0, x1);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  store_o((S - 1) / CT * CT, buf ^ 1);
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Sp[(int64_t)(32 * i + e) * dv] = st[4 * i + e];
+  // the convolution state: the last K-1 inputs (from the sequence, or shifted from the state when
+  // the sequence is shorter), in ascending slots so an in-place shift reads before it writes; the
+  // slice's v channels, and its share of the q and k channels of key head h
+  T* cst = static_cast<T*>(a.conv) + (int64_t)bb * (K - 1) * conv_dim;
+  const T* qs = static_cast<const T*>(a.qkv) + (int64_t)bb * S * a.qkv_stride;
+  auto advance = [&](int c) {
+    for (int i = 0; i < K - 1; ++i) {
+      const int u = S - (K - 1) + i;
+      cst[(int64_t)i * conv_dim + c] = u < 0 ? cst[(int64_t)(K - 1 + u) * conv_dim + c] : qs[(int64_t)u * a.qkv_stride + c];
+    }
+  };
+  if (tid < kGdnCols) advance(vch + tid);
+  if (h < Hk)
+    for (int i = slice * 256 + tid; i < 2 * DK; i += ns * 256) advance((i < DK ? 0 : key_dim - DK) + h * DK + i);
+}
+
+// Gated RMSNorm of the recurrence's outputs (in the v slots of `work`): a wave per (token, head).
+template <int DT>
+__global__ void __launch_bounds__(256) gdn_out_seq_kernel(GdnArgs a) {
+  using E = Elem<DT>;
+  using T = typename E::T;
+  const int lane = threadIdx.x & 63, Hv = a.Hv, dv = a.dv, nj = dv >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= (int64_t)a.B * a.S * Hv) return;
+  const int64_t row = i / Hv;
+  const int h = (int)(i - row * Hv);
+  const float* o = a.work + row * (2 * a.Hk * a.dk + Hv * dv) + 2 * a.Hk * a.dk + h * dv + lane;
+  const T* z = static_cast<const T*>(a.z) + row * a.z_stride + h * dv + lane;
+  const T* w = static_cast<const T*>(a.norm_w) + lane;
+  float ov[4], zv[4], wv[4], ss = 0.f;  // dv <= 256
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    ov[j] = j < nj ? o[64 * j] : 0.f;
+    zv[j] = j < nj ? E::ld(z + 64 * j) : 0.f;
+    wv[j] = j < nj ? E::ld(w + 64 * j) : 0.f;
+    ss += ov[j] * ov[j];
+  }
+  const float rn = 1.f / sqrtf(wave_sum(ss) / (float)dv + a.eps);
+  T* out = static_cast<T*>(a.out) + row * a.out_stride + h * dv + lane;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (j < nj) out[64 * j] = E::mk(ov[j] * rn * wv[j] * silu_f(zv[j]));
+}
+
+template <int DT>
+static hipError_t launch_gdn_seq_t(const GdnArgs& a, hipStream_t s) {
+  using T = typename Elem<DT>::T;
+  const int conv_dim = 2 * a.Hk * a.dk + a.Hv * a.dv;
+  // the column-split kernels: rows per lane in whole float4s of 8 lanes, a key head within one
+  // wave of the convolution, 16-byte pieces of `work`
+  if ((a.dk == 32 || a.dk == 64 || a.dk == 128) && (reinterpret_cast<uintptr_t>(a.work) & 15) == 0) {
+    const bool pair = ((a.qkv_stride & 1) | (reinterpret_cast<uintptr_t>(a.qkv) & (2 * sizeof(T) - 1))) == 0;
+    const dim3 pgrid((unsigned)((conv_dim + 511) / 512), (unsigned)((a.S + kGdnPrepTokens - 1) / kGdnPrepTokens),
+                     (unsigned)a.B);
+    const dim3 cgrid((unsigned)(a.Hv * (a.dv / kGdnCols)), (unsigned)a.B);
+    const int64_t waves = (int64_t)a.B * a.S * a.Hv;
+    if (waves > (int64_t)0x7FFFFFFF * 4 - 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gdn_prep_seq_kernel<DT>, pgrid, dim3(256), 0, s, a, pair);
+    if (a.dk == 32) hipLaunchKernelGGL((gdn_cols_seq_kernel<DT, 1>), cgrid, dim3(256), 0, s, a);
+    else if (a.dk == 64) hipLaunchKernelGGL((gdn_cols_seq_kernel<DT, 2>), cgrid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((gdn_cols_seq_kernel<DT, 4>), cgrid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(gdn_out_seq_kernel<DT>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, a);
+    return hipGetLastError();
+  }
+  const dim3 cgrid((unsigned)((conv_dim + 255) / 256), (unsigned)a.S, (unsigned)a.B), rgrid((unsigned)a.Hv, (unsigned)a.B);
+  hipLaunchKernelGGL(gdn_conv_seq_kernel<DT>, cgrid, dim3(256), 0, s, a);
+  hipLaunchKernelGGL(gdn_rec_seq_kernel<DT>, rgrid, dim3((unsigned)(kGdnRowGroups * a.dv)), 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_gdn_seq(int dt, const GdnArgs& a, hipStream_t s) {
+  if (dt == MD_F16) return launch_gdn_seq_t<MD_F16>(a, s);
+  if (dt == MD_BF16) return launch_gdn_seq_t<MD_BF16>(a, s);
+  return launch_gdn_seq_t<MD_F32>(a, s);
 }
 
 // ---- gated attention, one new token -------------------------------------------------------
