@@ -190,6 +190,10 @@ int resolve(int qt, DevTables* tb, int* num_cus, hipStream_t s = nullptr, bool m
 // largest tile plan), and one arrival counter per CU.
 long long qmm_ws_part_bytes(int num_cus) { return 2ll * num_cus * 256 * 256 * (long long)sizeof(float); }
 
+// Staging area for activations converted to fp16: 3855 rows of the 27B model's widest product
+// (K = 17408) at a time.
+constexpr long long kQmmStageBytes = 128ll << 20;
+
 // The QMM workspace of stream `s` on the current device, allocated on the first QMM call on
 // that stream (or by gsq_prepare); counters start at zero and every launch leaves them at zero.
 int qmm_workspace(hipStream_t s, QmmWorkspace* ws) {
@@ -225,7 +229,13 @@ int qmm_workspace(hipStream_t s, QmmWorkspace* ws) {
     if (cnt) hipFree(cnt);
     return fail(GSQ_E_HIP, "QMM workspace setup: %s", hipGetErrorString(e));
   }
-  *ws = st.qmm_ws[s] = QmmWorkspace{part, cnt, groups, part_bytes};
+  // the activation staging area is not required (the generic kernel runs without it)
+  void* xs = nullptr;
+  if (hipMalloc(&xs, (size_t)kQmmStageBytes) != hipSuccess) {
+    xs = nullptr;
+    (void)hipGetLastError();
+  }
+  *ws = st.qmm_ws[s] = QmmWorkspace{part, cnt, groups, part_bytes, xs, xs ? kQmmStageBytes : 0};
   return GSQ_OK;
 }
 

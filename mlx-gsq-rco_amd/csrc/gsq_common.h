@@ -171,6 +171,8 @@ struct QmmWorkspace {
   int* cnt;
   int max_groups;
   long long part_bytes;
+  void* xs = nullptr;      // fp16 staging of activations the MFMA kernels cannot read, or null
+  long long xs_bytes = 0;
 };
 
 // Non-linear IQ4_XS values (k_decode.py:77).

@@ -1,0 +1,49 @@
+"""Activations that ``gsq_qmm`` stages as fp16 (fp32, bf16, fp16 not 16-byte aligned): the result is
+that of the product on the same values as aligned fp16, bit for bit, over both fp16 kernels'
+ranges, and in pieces when the rows exceed the staging area."""
+import pytest
+import torch
+
+from mlx_gsq_amd import synth, tables
+
+pytestmark = pytest.mark.gpu
+if not torch.cuda.is_available():
+    pytest.skip("no GPU", allow_module_level=True)
+
+
+def _call(qtype, packed, x, m, n, k, code):
+    from mlx_gsq_amd import _lib
+    from mlx_gsq_amd.formats import TYPE_IDS
+    y = torch.full((m, n), float("nan"), device="cuda")
+    rc = _lib.lib().gsq_qmm(TYPE_IDS[qtype], packed.data_ptr(), x.data_ptr(), code, y.data_ptr(), 0, m, n, k,
+                            torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.lib().gsq_last_error()
+    return y
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 65, 300])
+@pytest.mark.parametrize("form", ["bf16", "fp32", "bf16+1", "fp32+1", "fp16+1"])
+@pytest.mark.parametrize("qtype,n,k", [("Q4_K", 515, 768), ("IQ3_S", 64, 256)])
+def test_staged_matches_fp16(qtype, n, k, form, m):
+    from mlx_gsq_amd import _lib
+    tables.set_tables(tables.synthetic_tables(0))
+    _lib.ensure_tables(qtype, torch.device("cuda:0"))
+    packed = torch.from_numpy(synth.make_packed(qtype, n, k, seed=1)).cuda()
+    dtype = {"bf16": torch.bfloat16, "fp32": torch.float32, "fp16": torch.float16}[form[:4]]
+    off = 1 if form.endswith("+1") else 0  # one element past an aligned address
+    x = torch.randn(m * k + 1, generator=torch.Generator().manual_seed(m)).to(dtype).cuda()[off:off + m * k]
+    assert (x.data_ptr() % 16 != 0) == bool(off)
+    want = _call(qtype, packed, x.half().clone(), m, n, k, 1)
+    got = _call(qtype, packed, x, m, n, k, _lib.DTYPE_CODES[dtype])
+    assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
+def test_rows_beyond_the_staging_area():
+    """128 MB of fp16 staging hold 3855 rows of K = 17408: 4000 rows go in two pieces of 2048 and 1952."""
+    m, n, k = 4000, 40, 17408
+    packed = torch.from_numpy(synth.make_packed("Q4_K", n, k, seed=2)).cuda()
+    x = torch.randn(m, k, device="cuda", generator=torch.Generator("cuda").manual_seed(3)).bfloat16()
+    got = _call("Q4_K", packed, x, m, n, k, 2)
+    h = x.half()
+    want = torch.cat([_call("Q4_K", packed, h[a:b], b - a, n, k, 1) for a, b in ((0, 2048), (2048, 4000))])
+    assert torch.isfinite(got).all() and torch.equal(got, want)
