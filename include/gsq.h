@@ -214,6 +214,19 @@ int gsq_attn_decode(const void* qg, int64_t qg_stride, const void* k, int64_t k_
                     int64_t heads, int64_t kv_heads, int64_t head_dim, int64_t rotary_dim, int64_t max_len,
                     float eps, float* work, int64_t chunk, int dtype, void* stream);
 
+/* gsq_attn_decode for a prompt: `seq` new tokens of each of `batch` rows at positions *pos ..
+ * *pos + seq - 1, rows b * seq + t of qg, k, v and out; token t attends to positions 0 .. *pos + t
+ * (the caches before, the new tokens up to itself). Same arithmetic and roundings per token: scores,
+ * softmax and the sums over V at fp32 accuracy. fp16 or bf16; head_dim 64, 128 or 256; caches and
+ * q_work (batch * heads * seq * head_dim values of scratch) 16-byte aligned, rows of qg and out
+ * 8-byte aligned. When the tokens do not all lie inside the cache the kernels write NaN to out and
+ * nothing to the caches. */
+int gsq_attn_seq(const void* qg, int64_t qg_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
+                 const void* q_norm_w, const void* k_norm_w, const double* inv_freq, void* k_cache, void* v_cache,
+                 const int64_t* pos, void* out, int64_t out_stride, void* q_work, int64_t batch, int64_t seq,
+                 int64_t heads, int64_t kv_heads, int64_t head_dim, int64_t rotary_dim, int64_t max_len, float eps,
+                 int dtype, void* stream);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char* gsq_last_error(void);
 

@@ -33,6 +33,7 @@ hipError_t launch_add_rms_norm(int dt, void* x, const void* delta, const void* w
 hipError_t launch_swiglu(int dt, const void* gu, void* out, int64_t rows, int n, hipStream_t s);
 hipError_t launch_gdn_step(int dt, const GdnArgs& a, hipStream_t s);
 hipError_t launch_gdn_seq(int dt, const GdnArgs& a, hipStream_t s);
+hipError_t launch_attn_seq(bool bf16, const AttnSeqArgs& a, hipStream_t s);
 hipError_t launch_attn_decode(int dt, const AttnArgs& a, hipStream_t s);
 int qmv_table_bytes(int qt);
 int build_qmv_table(int qt, const uint16_t* grid16, const uint8_t* ksigns, std::vector<uint8_t>& out);
@@ -691,6 +692,41 @@ int gsq_attn_decode(const void* qg, int64_t qg_stride, const void* k, int64_t k_
   }
   hipError_t e = launch_attn_decode(dtype, a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(GSQ_E_HIP, "attn_decode launch: %s", hipGetErrorString(e));
+  return GSQ_OK;
+}
+
+int gsq_attn_seq(const void* qg, int64_t qg_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
+                 const void* q_norm_w, const void* k_norm_w, const double* inv_freq, void* k_cache, void* v_cache,
+                 const int64_t* pos, void* out, int64_t out_stride, void* q_work, int64_t batch, int64_t seq,
+                 int64_t heads, int64_t kv_heads, int64_t head_dim, int64_t rotary_dim, int64_t max_len, float eps,
+                 int dtype, void* stream) {
+  if (dtype != GSQ_F16 && dtype != GSQ_BF16) return fail(GSQ_E_TYPE, "unsupported dtype code %d", dtype);
+  if (batch < 0 || batch > 65535 || seq < 0) return fail(GSQ_E_VALUE, "batch must be 0..65535, seq not negative");
+  if (batch == 0 || seq == 0) return GSQ_OK;
+  if (kv_heads <= 0 || heads <= 0 || heads % kv_heads || heads > 65535)
+    return fail(GSQ_E_VALUE, "heads must be a positive multiple of kv heads (at most 65535)");
+  if (head_dim != 64 && head_dim != 128 && head_dim != 256) return fail(GSQ_E_VALUE, "head dim must be 64, 128 or 256");
+  if (rotary_dim < 0 || rotary_dim > head_dim || rotary_dim % 2) return fail(GSQ_E_VALUE, "invalid rotary dim");
+  if (max_len <= 0 || max_len >= (1ll << 31) - 64) return fail(GSQ_E_VALUE, "invalid cache length");
+  if (seq > max_len) return fail(GSQ_E_VALUE, "%lld tokens do not fit a cache of %lld", (long long)seq, (long long)max_len);
+  if ((seq + 63) / 64 * heads >= (1ll << 31)) return fail(GSQ_E_VALUE, "too many query tiles");
+  if (!qg || !k || !v || !q_norm_w || !k_norm_w || (!inv_freq && rotary_dim) || !k_cache || !v_cache || !pos || !out ||
+      !q_work)
+    return fail(GSQ_E_VALUE, "NULL pointer");
+  if ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) |
+       reinterpret_cast<uintptr_t>(q_work)) & 15)
+    return fail(GSQ_E_VALUE, "k_cache, v_cache and q_work must be 16-byte aligned");
+  if (((reinterpret_cast<uintptr_t>(qg) | reinterpret_cast<uintptr_t>(out)) & 7) || qg_stride % 4 || out_stride % 4)
+    return fail(GSQ_E_VALUE, "rows of qg and out must be 8-byte aligned");
+  if (!(eps >= 0.f)) return fail(GSQ_E_VALUE, "eps must be >= 0");
+  AttnSeqArgs a;
+  a.qg = qg; a.k = k; a.v = v; a.q_norm_w = q_norm_w; a.k_norm_w = k_norm_w; a.inv_freq = inv_freq;
+  a.kc = k_cache; a.vc = v_cache; a.pos = pos; a.q = q_work; a.out = out;
+  a.qg_stride = qg_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.out_stride = out_stride;
+  a.B = (int)batch; a.S = (int)seq; a.H = (int)heads; a.Hkv = (int)kv_heads; a.hd = (int)head_dim;
+  a.rd = (int)rotary_dim; a.L = (int)max_len; a.eps = eps;
+  hipError_t e = launch_attn_seq(dtype == GSQ_BF16, a, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(GSQ_E_HIP, "attn_seq launch: %s", hipGetErrorString(e));
   return GSQ_OK;
 }
 

@@ -162,6 +162,25 @@ struct AttnArgs {
   int chunk = 0, nsplit = 0;
 };
 
+// Arguments of the gated attention of S new tokens per batch row (gsq_attn_seq; kernels in
+// gsq_attn_seq.hip), at positions pos .. pos + S - 1 of the caches. Rows b * S + t of qg, k, v, out.
+struct AttnSeqArgs {
+  const void* qg;  // rows of H * 2hd: per head q then gate (row stride qg_stride)
+  const void* k;   // rows of Hkv * hd
+  const void* v;
+  const void* q_norm_w;  // [hd]
+  const void* k_norm_w;
+  const double* inv_freq;  // [rd / 2]
+  void* kc;  // [B, Hkv, L, hd]
+  void* vc;
+  const int64_t* pos;  // position of the first new token (device)
+  void* q;    // scratch [B, H, S, hd]: normalized, rotated queries
+  void* out;  // rows of H * hd
+  int64_t qg_stride, k_stride, v_stride, out_stride;
+  int B, S, H, Hkv, hd, rd, L;
+  float eps;
+};
+
 // QMM workspace: fp32 partial tiles of workgroups that share an output tile (2 slots per
 // workgroup, each sized to the launch plan's tile) and one arrival counter per workgroup, kept
 // at zero between launches. `part_bytes` bounds 2 * groups * slot bytes; `max_groups` bounds the

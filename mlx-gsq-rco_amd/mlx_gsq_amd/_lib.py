@@ -39,6 +39,8 @@ EXPORTS = {
     "gsq_swiglu": (_I32, [_VP, _VP, _I64, _I64, _I32, _VP]),
     "gsq_attn_decode": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64,
                                _I64, _I64, _I64, _I64, _F32, _VP, _I64, _I32, _VP]),
+    "gsq_attn_seq": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP, _I64, _I64,
+                            _I64, _I64, _I64, _I64, _I64, _F32, _I32, _VP]),
     "gsq_gdn_step": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64,
                             _VP, _I64, _I64, _I64, _I64, _I64, _I64, _F32, _I32, _VP]),
     "gsq_gdn_seq": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP, _I64,

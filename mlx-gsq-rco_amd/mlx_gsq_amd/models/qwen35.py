@@ -263,6 +263,16 @@ class FullAttention(torch.nn.Module):
         """qk_proj of the row its prologue forms from x (``forward_pre`` keywords)."""
         return self.qk_proj.forward_pre(x, "add_rms_norm", **kw)
 
+    def _seq_kernel(self, qk, v, cache) -> bool:
+        """Whether the prompt kernel takes these tensors: one 16-bit dtype throughout, a head dim it
+        is built for, contiguous rows at its alignments; the torch formulation runs otherwise."""
+        from ..runtime.kernels.model_ops import ATTN_SEQ_HEAD_DIMS
+        a_ = self.args
+        kc, vc = cache.k[self.layer], cache.v[self.layer]
+        return (qk.dtype in (torch.float16, torch.bfloat16) and a_.head_dim in ATTN_SEQ_HEAD_DIMS
+                and all(t.dtype == qk.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (qk, v, kc, vc))
+                and self.q_norm_w.dtype == self.k_norm_w.dtype == qk.dtype and qk.shape[1] <= kc.shape[2])
+
     def forward(self, x, cache: Qwen35Cache, first=None):
         """``first``: ``qk_proj(x)`` when the caller has computed it already."""
         a_ = self.args
@@ -277,6 +287,12 @@ class FullAttention(torch.nn.Module):
                                         cache.pos, heads=H, kv_heads=Hkv, head_dim=hd, rotary_dim=a_.rotary_dim,
                                         eps=a_.rms_norm_eps)
             return self.o_proj(out.view(B, 1, H * hd))
+        if x.is_cuda and self._seq_kernel(qk, v, cache):
+            from ..runtime.kernels import model_ops
+            out = model_ops.attn_seq(qk[..., :H * 2 * hd], qk[..., H * 2 * hd:], v, self.q_norm_w, self.k_norm_w,
+                                     self.inv_freq, cache.k[self.layer], cache.v[self.layer], cache.pos, heads=H,
+                                     kv_heads=Hkv, head_dim=hd, rotary_dim=a_.rotary_dim, eps=a_.rms_norm_eps)
+            return self.o_proj(out)
         qg = qk[..., :H * 2 * hd].reshape(B, S, H, 2 * hd)
         q, gate = qg[..., :hd], qg[..., hd:].reshape(B, S, H * hd)
         q = rms_norm(q, self.q_norm_w, a_.rms_norm_eps)

@@ -185,3 +185,41 @@ def attn_decode(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos, *
             L, float(eps), None if work is None else work.data_ptr(), int(chunk), _dt(qg),
             _lib.stream_handle(dev)), "attn_decode")
     return out
+
+
+ATTN_SEQ_HEAD_DIMS = (64, 128, 256)
+
+
+def attn_seq(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos, *, heads: int, kv_heads: int,
+             head_dim: int, rotary_dim: int, eps: float):
+    """``attn_decode`` for a prompt: S new tokens of B rows at positions pos .. pos + S - 1; qg
+    (B, S, heads * 2 head_dim), k and v (B, S, kv_heads * head_dim) with unit inner stride and the
+    (B, S) rows at one stride each, fp16 or bf16, head_dim 64, 128 or 256. Returns
+    (B, S, heads * head_dim)."""
+    dev = _on_gpu(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos)
+    B, S = qg.shape[0], qg.shape[1]
+    if qg.dtype not in (torch.float16, torch.bfloat16):
+        raise TypeError(f"unsupported dtype {qg.dtype}")
+    for t in (qg, k, v):
+        if (t.dim() != 3 or tuple(t.shape[:2]) != (B, S) or t.stride(2) != 1 or t.dtype != qg.dtype
+                or (B > 1 and t.stride(0) != S * t.stride(1))):
+            raise ValueError("qg, k and v must be (B, S, n) of one dtype, unit inner stride, rows at one stride")
+    if (qg.shape[2] != heads * 2 * head_dim or k.shape[2] != kv_heads * head_dim or v.shape[2] != kv_heads * head_dim
+            or q_norm_w.numel() != head_dim or k_norm_w.numel() != head_dim or inv_freq.numel() != rotary_dim // 2
+            or k_cache.shape != v_cache.shape or tuple(k_cache.shape[:2]) != (B, kv_heads)
+            or k_cache.shape[3] != head_dim):
+        raise ValueError("attention tensor shapes do not match the head configuration")
+    if inv_freq.dtype != torch.float64 or pos.dtype != torch.int64 or pos.numel() != 1:
+        raise ValueError("inv_freq must be float64 and pos one int64")
+    for t in (q_norm_w, k_norm_w, k_cache, v_cache):
+        if t.dtype != qg.dtype or not t.is_contiguous():
+            raise ValueError("norm weights and caches must be contiguous in the activation dtype")
+    out = torch.empty(B, S, heads * head_dim, dtype=qg.dtype, device=dev)
+    work = torch.empty(B * heads * S * head_dim, dtype=qg.dtype, device=dev)
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().gsq_attn_seq(
+            qg.data_ptr(), qg.stride(1), k.data_ptr(), k.stride(1), v.data_ptr(), v.stride(1), q_norm_w.data_ptr(),
+            k_norm_w.data_ptr(), inv_freq.contiguous().data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+            pos.data_ptr(), out.data_ptr(), out.stride(1), work.data_ptr(), B, S, heads, kv_heads, head_dim,
+            rotary_dim, k_cache.shape[2], float(eps), _dt(qg), _lib.stream_handle(dev)), "attn_seq")
+    return out
