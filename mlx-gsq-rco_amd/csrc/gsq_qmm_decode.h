@@ -94,81 +94,123 @@ __device__ __forceinline__ const uint32_t* tbl_words(const uint8_t* tbl, uint32_
   return reinterpret_cast<const uint32_t*>(tbl + byte_off);
 }
 
+// Words at a byte offset of an LDS row slot, read now and shifted into place later: the loads can be
+// issued well before their first use (load() and get() on either side of other work).
+template <int N, bool A4>
+struct LdsWords {
+  uint32_t a[A4 ? N : N + 1], sh;
+  __device__ __forceinline__ void load(const uint8_t* base, uint32_t off) {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(base + (A4 ? off : off & ~3u));
+    sh = off & 3u;
+#pragma unroll
+    for (int i = 0; i < (A4 ? N : N + 1); ++i) a[i] = p[i];
+  }
+  __device__ __forceinline__ uint32_t get(int i) const {
+    if constexpr (A4) return a[i];
+    else return __builtin_amdgcn_alignbyte(a[i + 1], a[i], sh);
+  }
+};
+
+// QmmDec<T>::run decodes one fragment slice. The caller's `after_fields` and `after_lookups` run
+// between its three phases (superblock field reads; codebook and mask reads; arithmetic), so that
+// other work can cover the LDS latency of each: the tiled kernel issues MFMAs there.
+struct QmmNoWork {
+  __device__ __forceinline__ void operator()() const {}
+};
+
 template <int T, bool A4>
 struct QmmDec;
+
+#define GSQ_QMM_RUN                                                                                              \
+  template <class F1 = QmmNoWork, class F2 = QmmNoWork>                                                          \
+  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq,  \
+                                             uint32_t (&o)[4], F1 after_fields = F1{}, F2 after_lookups = F2{})
 
 // Q2_K (k_decode.py:18-30): w = d*(sm&15)*q - dmin*(sm>>4)
 template <bool A4>
 struct QmmDec<Q2_K, A4> {
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t*, int g, int kq, uint32_t (&o)[4]) {
-    uint32_t q[2];
-    lds_words<2, A4>(sb, sd + 16 + (g >> 2) * 32 + 8 * kq, q);
-    const int sh = 2 * (g & 3);
-    q[0] = (q[0] >> sh) & 0x03030303u;
-    q[1] = (q[1] >> sh) & 0x03030303u;
-    const uint32_t dd = lds_w32<A4>(sb, sd + 80);
+  GSQ_QMM_RUN {
+    LdsWords<2, A4> qw;
+    LdsWords<1, A4> dw;
+    qw.load(sb, sd + 16 + (g >> 2) * 32 + 8 * kq);
+    dw.load(sb, sd + 80);
     const uint32_t sm = lds_u8(sb, sd + 2 * g + (kq >> 1));
+    after_fields();
+    const int sh = 2 * (g & 3);
+    const uint32_t q[2] = {(qw.get(0) >> sh) & 0x03030303u, (qw.get(1) >> sh) & 0x03030303u};
+    const uint32_t dd = dw.get(0);
     const float a = h2f(dd & 0xFFFFu) * (float)(sm & 15u);
     const float b = h2f(dd >> 16) * (float)(sm >> 4);
+    after_lookups();
     codes8(q, a * kCode, -b, o);
+    (void)tbl;
   }
 };
 
 // Q4_K (k_decode.py:31-50): w = d*sc*q - dmin*mn with 6-bit scales/mins
 template <bool A4>
 struct QmmDec<Q4_K, A4> {
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t*, int g, int kq, uint32_t (&o)[4]) {
-    uint32_t q[2];
-    lds_words<2, A4>(sb, sd + 16 + (g >> 1) * 32 + 8 * kq, q);
+  GSQ_QMM_RUN {
+    LdsWords<2, A4> qw;
+    LdsWords<4, A4> dw;  // d | dmin, then the 12 scale bytes
+    qw.load(sb, sd + 16 + (g >> 1) * 32 + 8 * kq);
+    dw.load(sb, sd);
+    after_fields();
     const int sh = 4 * (g & 1);
-    q[0] = (q[0] >> sh) & 0x0F0F0F0Fu;
-    q[1] = (q[1] >> sh) & 0x0F0F0F0Fu;
-    uint32_t s[3];
-    lds_words<3, A4>(sb, sd + 4, s);
-    const uint32_t dd = lds_w32<A4>(sb, sd + 0);
+    const uint32_t q[2] = {(qw.get(0) >> sh) & 0x0F0F0F0Fu, (qw.get(1) >> sh) & 0x0F0F0F0Fu};
+    const uint32_t dd = dw.get(0);
     uint32_t sc, mn;
     const int gg = g & 3;
     if (g < 4) {
-      sc = bfe(s[0], 8 * gg, 6);
-      mn = bfe(s[1], 8 * gg, 6);
+      sc = bfe(dw.get(1), 8 * gg, 6);
+      mn = bfe(dw.get(2), 8 * gg, 6);
     } else {
-      const uint32_t lo = bfe(s[2], 8 * gg, 8);
-      sc = (lo & 15u) | (bfe(s[0], 8 * gg + 6, 2) << 4);
-      mn = (lo >> 4) | (bfe(s[1], 8 * gg + 6, 2) << 4);
+      const uint32_t lo = bfe(dw.get(3), 8 * gg, 8);
+      sc = (lo & 15u) | (bfe(dw.get(1), 8 * gg + 6, 2) << 4);
+      mn = (lo >> 4) | (bfe(dw.get(2), 8 * gg + 6, 2) << 4);
     }
     const float a = h2f(dd & 0xFFFFu) * (float)sc;
     const float b = h2f(dd >> 16) * (float)mn;
+    after_lookups();
     codes8(q, a * kCode, -b, o);
+    (void)tbl;
   }
 };
 
 // Q6_K (k_decode.py:51-65): w = d*scale*(q - 32), q = low nibble | 2 high bits << 4
 template <bool A4>
 struct QmmDec<Q6_K, A4> {
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t*, int g, int kq, uint32_t (&o)[4]) {
+  GSQ_QMM_RUN {
     const int h = g >> 2, pl = g & 3;
     uint32_t ql[2], qh[2];
     lds_words<2, A4>(sb, sd + h * 64 + (pl & 1) * 32 + 8 * kq, ql);
     lds_words<2, A4>(sb, sd + 128 + h * 32 + 8 * kq, qh);
+    after_fields();
     const int shl = 4 * (pl >> 1), shh = 2 * pl;
     uint32_t q[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) q[i] = ((ql[i] >> shl) & 0x0F0F0F0Fu) | (((qh[i] >> shh) & 0x03030303u) << 4);
     const int sc = (int)(int8_t)lds_u8(sb, sd + 192 + 2 * g + (kq >> 1));
     const float a = h2f(lds_u16(sb, sd + 208)) * (float)sc;
+    after_lookups();
     codes8(q, a * kCode, -32.f * a, o);
+    (void)tbl;
   }
 };
 
 // IQ4_XS (k_decode.py:66-80): w = d*scale*kvalues[q]; kvalues + 128 looked up as bytes
 template <bool A4>
 struct QmmDec<IQ4_XS, A4> {
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t*, int g, int kq, uint32_t (&o)[4]) {
-    uint32_t q[2];
-    lds_words<2, A4>(sb, sd + 8 + 16 * g + 8 * (kq & 1), q);
+  GSQ_QMM_RUN {
+    LdsWords<2, A4> qw;
+    LdsWords<1, A4> dww;
+    qw.load(sb, sd + 8 + 16 * g + 8 * (kq & 1));
+    dww.load(sb, sd);
+    const uint32_t slow = lds_u8(sb, sd + 4 + g / 2);
+    after_fields();
     const int sh = 4 * (kq >> 1);
-    const uint32_t dw = lds_w32<A4>(sb, sd + 0);
-    const uint32_t low = (lds_u8(sb, sd + 4 + g / 2) >> (4 * (g & 1))) & 15u;
+    const uint32_t dw = dww.get(0);
+    const uint32_t low = (slow >> (4 * (g & 1))) & 15u;
     const uint32_t high = ((dw >> 16) >> (2 * g)) & 3u;
     const float a = h2f(dw & 0xFFFFu) * (float)((int)(low | (high << 4)) - 32);
     // kvalues + 128 = {1,24,45,63,79,93,106,118,129,141,153,166,181,197,217,241}
@@ -176,14 +218,16 @@ struct QmmDec<IQ4_XS, A4> {
     uint32_t u[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const uint32_t c = (q[i] >> sh) & 0x0F0F0F0Fu;
+      const uint32_t c = (qw.get(i) >> sh) & 0x0F0F0F0Fu;
       const uint32_t sel = c & 0x07070707u;
       const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel);
       const uint32_t hi = __builtin_amdgcn_perm(T3, T2, sel);
       const uint32_t m = ((c >> 3) & 0x01010101u) * 0xFFu;
       u[i] = (hi & m) | (lo & ~m);
     }
+    after_lookups();
     codes8(u, a * kCode, -128.f * a, o);
+    (void)tbl;
   }
 };
 
@@ -193,45 +237,28 @@ template <bool A4>
 struct QmmDec<IQ3_S, A4> {
   static constexpr uint32_t kGridB = 512 * 4 * 2;
   static constexpr uint32_t kMaskB = kGridB;
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
-    const float d = h2f(lds_u16(sb, sd + 0));
+  GSQ_QMM_RUN {
+    const uint32_t dh = lds_u16(sb, sd + 0);
     const uint32_t sbyte = lds_u8(sb, sd + 106 + (g >> 1));
-    const float db = d * (float)(1u + 2u * ((sbyte >> (4 * (g & 1))) & 15u));
     const uint32_t qh = lds_u8(sb, sd + 66 + g);
     const uint32_t qq = lds_u16(sb, sd + 2 + 8 * g + 2 * kq);
+    const uint32_t signs = lds_u8(sb, sd + 74 + 4 * g + kq);
+    after_fields();
     const uint32_t i0 = (qq & 0xFFu) | ((qh << (8 - 2 * kq)) & 256u);
     const uint32_t i1 = (qq >> 8) | ((qh << (7 - 2 * kq)) & 256u);
-    const uint32_t signs = lds_u8(sb, sd + 74 + 4 * g + kq);
-    const uint32_t* e0 = tbl_words(tbl, i0 * 8);
-    const uint32_t* e1 = tbl_words(tbl, i1 * 8);
     // nibble masks (16 entries: few distinct LDS addresses per read, unlike the 256 byte masks)
-    const uint32_t* m0 = tbl_words(tbl, kMaskB + (signs & 15u) * 8);
-    const uint32_t* m1 = tbl_words(tbl, kMaskB + (signs >> 4) * 8);
-    o[0] = mix2(db, e0[0], 0.f) ^ m0[0];
-    o[1] = mix2(db, e0[1], 0.f) ^ m0[1];
-    o[2] = mix2(db, e1[0], 0.f) ^ m1[0];
-    o[3] = mix2(db, e1[1], 0.f) ^ m1[1];
+    const uint2 e0 = *reinterpret_cast<const uint2*>(tbl + i0 * 8);
+    const uint2 e1 = *reinterpret_cast<const uint2*>(tbl + i1 * 8);
+    const uint2 m0 = *reinterpret_cast<const uint2*>(tbl + kMaskB + (signs & 15u) * 8);
+    const uint2 m1 = *reinterpret_cast<const uint2*>(tbl + kMaskB + (signs >> 4) * 8);
+    const float db = h2f(dh) * (float)(1u + 2u * ((sbyte >> (4 * (g & 1))) & 15u));
+    after_lookups();
+    o[0] = mix2(db, e0.x, 0.f) ^ m0.x;
+    o[1] = mix2(db, e0.y, 0.f) ^ m0.y;
+    o[2] = mix2(db, e1.x, 0.f) ^ m1.x;
+    o[3] = mix2(db, e1.y, 0.f) ^ m1.y;
   }
 };
-
-// one 8-wide codebook entry times d, with four sign-mask pairs (HM) or none; the entry and
-// mask words are read before any is used
-template <bool HM>
-__device__ __forceinline__ void grid8(const uint8_t* tbl, uint32_t qi, float d, float c, const uint32_t* m,
-                                      uint32_t (&o)[4]) {
-  const uint32_t* e = tbl_words(tbl, qi * 16);
-  uint32_t ev[4], mv[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) ev[i] = e[i];
-  if constexpr (HM) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mv[i] = m[i];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = mix2(d, ev[i], c) ^ mv[i];  // the XOR is the visible VALU write
-  } else {
-    mix8(d, ev, c, o);  // no sign masks: the asm block carries the MFMA wait states itself
-  }
-}
 
 // Sign masks of one ksigns field (8 weights, 4 words): the sign byte from the ksigns table's
 // closed form (entry i = i with bit 7 the parity of i; the library accepts no other table),
@@ -241,38 +268,64 @@ __device__ __forceinline__ void grid8(const uint8_t* tbl, uint32_t qi, float d, 
 // table in their images (the nibble form was 1-6% slower for them here).
 __device__ __forceinline__ void ksigns_masks(const uint8_t* tbl, uint32_t mask_off, uint32_t k7, uint32_t (&m)[4]) {
   const uint32_t s8 = k7 | ((__builtin_popcount(k7) & 1u) << 7);
-  const uint32_t* lo = tbl_words(tbl, mask_off + (s8 & 15u) * 8);
-  const uint32_t* hi = tbl_words(tbl, mask_off + (s8 >> 4) * 8);
-  m[0] = lo[0]; m[1] = lo[1]; m[2] = hi[0]; m[3] = hi[1];
+  const uint2 lo = *reinterpret_cast<const uint2*>(tbl + mask_off + (s8 & 15u) * 8);
+  const uint2 hi = *reinterpret_cast<const uint2*>(tbl + mask_off + (s8 >> 4) * 8);
+  m[0] = lo.x; m[1] = lo.y; m[2] = hi.x; m[3] = hi.y;
 }
 
 // IQ3_XXS (iq_lookup_decode.py:7-12): w = +-d*(0.5+s)*0.5*grid[qi][c], ksigns masks
 template <bool A4>
 struct QmmDec<IQ3_XXS, A4> {
   static constexpr uint32_t kGridB = 256 * 4 * 2;
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
-    const uint32_t u = lds_w32<A4>(sb, sd + 66 + 4 * g);
-    const float d = h2f(lds_u16(sb, sd + 0)) * (0.5f + (float)(u >> 28)) * 0.5f;
-    uint32_t m[4];
-    ksigns_masks(tbl, kGridB, (u >> (7 * kq)) & 127u, m);
+  GSQ_QMM_RUN {
+    LdsWords<1, A4> uw;
+    uw.load(sb, sd + 66 + 4 * g);
+    const uint32_t dh = lds_u16(sb, sd + 0);
     const uint32_t qq = lds_u16(sb, sd + 2 + 8 * g + 2 * kq);
-    const uint32_t* e0 = tbl_words(tbl, (qq & 0xFFu) * 8);
-    const uint32_t* e1 = tbl_words(tbl, (qq >> 8) * 8);
-    o[0] = mix2(d, e0[0], 0.f) ^ m[0];
-    o[1] = mix2(d, e0[1], 0.f) ^ m[1];
-    o[2] = mix2(d, e1[0], 0.f) ^ m[2];
-    o[3] = mix2(d, e1[1], 0.f) ^ m[3];
+    after_fields();
+    const uint32_t u = uw.get(0);
+    uint32_t m[4];
+    const uint2 e0 = *reinterpret_cast<const uint2*>(tbl + (qq & 0xFFu) * 8);
+    const uint2 e1 = *reinterpret_cast<const uint2*>(tbl + (qq >> 8) * 8);
+    ksigns_masks(tbl, kGridB, (u >> (7 * kq)) & 127u, m);
+    const float d = h2f(dh) * (0.5f + (float)(u >> 28)) * 0.5f;
+    after_lookups();
+    o[0] = mix2(d, e0.x, 0.f) ^ m[0];
+    o[1] = mix2(d, e0.y, 0.f) ^ m[1];
+    o[2] = mix2(d, e1.x, 0.f) ^ m[2];
+    o[3] = mix2(d, e1.y, 0.f) ^ m[3];
   }
 };
+
+// one 8-wide codebook entry times d, signs flipped by four mask pairs
+__device__ __forceinline__ void grid8(const uint4& e, const uint4& m, float d, uint32_t (&o)[4]) {
+  o[0] = mix2(d, e.x, 0.f) ^ m.x;  // the XOR is the visible VALU write
+  o[1] = mix2(d, e.y, 0.f) ^ m.y;
+  o[2] = mix2(d, e.z, 0.f) ^ m.z;
+  o[3] = mix2(d, e.w, 0.f) ^ m.w;
+}
+// ... without signs: the asm block carries the MFMA wait states itself
+__device__ __forceinline__ void grid8(const uint4& e, float d, uint32_t (&o)[4]) {
+  const uint32_t ev[4] = {e.x, e.y, e.z, e.w};
+  mix8(d, ev, 0.f, o);
+}
 
 // IQ2_XXS (iq_lookup_decode.py:23-26)
 template <bool A4>
 struct QmmDec<IQ2_XXS, A4> {
   static constexpr uint32_t kGridB = 256 * 8 * 2;
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
-    const uint32_t u = lds_w32<A4>(sb, sd + 2 + 8 * g + 4);
-    const float d = h2f(lds_u16(sb, sd + 0)) * (0.5f + (float)(u >> 28)) * 0.25f;
-    grid8<true>(tbl, lds_u8(sb, sd + 2 + 8 * g + kq), d, 0.f, tbl_words(tbl, kGridB + 16 * 8 + ((u >> (7 * kq)) & 127u) * 16), o);
+  GSQ_QMM_RUN {
+    LdsWords<1, A4> uw;
+    uw.load(sb, sd + 2 + 8 * g + 4);
+    const uint32_t dh = lds_u16(sb, sd + 0);
+    const uint32_t qi = lds_u8(sb, sd + 2 + 8 * g + kq);
+    after_fields();
+    const uint32_t u = uw.get(0);
+    const uint4 e = *reinterpret_cast<const uint4*>(tbl + qi * 16);
+    const uint4 m = *reinterpret_cast<const uint4*>(tbl + kGridB + 16 * 8 + ((u >> (7 * kq)) & 127u) * 16);
+    const float d = h2f(dh) * (0.5f + (float)(u >> 28)) * 0.25f;
+    after_lookups();
+    grid8(e, m, d, o);
   }
 };
 
@@ -280,11 +333,16 @@ struct QmmDec<IQ2_XXS, A4> {
 template <bool A4>
 struct QmmDec<IQ2_XS, A4> {
   static constexpr uint32_t kGridB = 512 * 8 * 2;
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
+  GSQ_QMM_RUN {
     const uint32_t q = lds_u16(sb, sd + 2 + 2 * (4 * g + kq));
-    const uint32_t sc = (lds_u8(sb, sd + 66 + g) >> (4 * (kq >> 1))) & 15u;
-    const float d = h2f(lds_u16(sb, sd + 0)) * (0.5f + (float)sc) * 0.25f;
-    grid8<true>(tbl, q & 511u, d, 0.f, tbl_words(tbl, kGridB + 16 * 8 + (q >> 9) * 16), o);
+    const uint32_t scb = lds_u8(sb, sd + 66 + g);
+    const uint32_t dh = lds_u16(sb, sd + 0);
+    after_fields();
+    const uint4 e = *reinterpret_cast<const uint4*>(tbl + (q & 511u) * 16);
+    const uint4 m = *reinterpret_cast<const uint4*>(tbl + kGridB + 16 * 8 + (q >> 9) * 16);
+    const float d = h2f(dh) * (0.5f + (float)((scb >> (4 * (kq >> 1))) & 15u)) * 0.25f;
+    after_lookups();
+    grid8(e, m, d, o);
   }
 };
 
@@ -292,18 +350,20 @@ struct QmmDec<IQ2_XS, A4> {
 template <bool A4>
 struct QmmDec<IQ2_S, A4> {
   static constexpr uint32_t kGridB = 1024 * 8 * 2;
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
+  GSQ_QMM_RUN {
     const int oo = 4 * g + kq;
     const uint32_t hi = (lds_u8(sb, sd + 66 + g) >> (2 * kq)) & 3u;
     const uint32_t qi = lds_u8(sb, sd + 2 + oo) | (hi << 8);
     const uint32_t sc = (lds_u8(sb, sd + 74 + g) >> (4 * (kq >> 1))) & 15u;
     const float d = h2f(lds_u16(sb, sd + 0)) * (0.5f + (float)sc) * 0.25f;
     const uint32_t sg = lds_u8(sb, sd + 34 + oo);
+    after_fields();
     const uint32_t* e = tbl_words(tbl, qi * 16);
     const uint32_t* m0 = tbl_words(tbl, kGridB + (sg & 15u) * 8);
     const uint32_t* m1 = tbl_words(tbl, kGridB + (sg >> 4) * 8);
     const uint32_t ev[4] = {e[0], e[1], e[2], e[3]};
     const uint32_t mv[4] = {m0[0], m0[1], m1[0], m1[1]};
+    after_lookups();
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = mix2(d, ev[i], 0.f) ^ mv[i];
   }
@@ -313,11 +373,16 @@ struct QmmDec<IQ2_S, A4> {
 // grid + delta (entry qi | 2048 for delta = -0.125, the sign bit 15 of qh)
 template <bool A4>
 struct QmmDec<IQ1_S, A4> {
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
+  GSQ_QMM_RUN {
     const uint32_t h = lds_u16(sb, sd + 34 + 2 * g);
-    const float d = h2f(lds_u16(sb, sd + 0)) * (float)(2u * ((h >> 12) & 7u) + 1u);
-    const uint32_t qi = lds_u8(sb, sd + 2 + 4 * g + kq) | (((h >> (3 * kq)) & 7u) << 8) | ((h >> 15) << 11);
-    grid8<false>(tbl, qi, d, 0.f, nullptr, o);
+    const uint32_t dh = lds_u16(sb, sd + 0);
+    const uint32_t ql = lds_u8(sb, sd + 2 + 4 * g + kq);
+    after_fields();
+    const uint32_t qi = ql | (((h >> (3 * kq)) & 7u) << 8) | ((h >> 15) << 11);
+    const uint4 e = *reinterpret_cast<const uint4*>(tbl + qi * 16);
+    const float d = h2f(dh) * (float)(2u * ((h >> 12) & 7u) + 1u);
+    after_lookups();
+    grid8(e, d, o);
   }
 };
 
@@ -326,21 +391,27 @@ struct QmmDec<IQ1_S, A4> {
 // = delta's sign)
 template <bool A4>
 struct QmmDec<IQ1_M, A4> {
-  __device__ __forceinline__ static void run(const uint8_t* sb, uint32_t sd, const uint8_t* tbl, int g, int kq, uint32_t (&o)[4]) {
-    uint32_t w[2];
-    lds_words<2, A4>(sb, sd + 48, w);
-    const uint32_t w0 = w[0] & 0xFFFFu, w1 = w[0] >> 16, w2 = w[1] & 0xFFFFu, w3 = w[1] >> 16;
-    const uint32_t dbits = ((w0 & 61440u) >> 12) | ((w1 & 61440u) >> 8) | ((w2 & 61440u) >> 4) | (w3 & 61440u);
+  GSQ_QMM_RUN {
+    LdsWords<2, A4> ww;
+    ww.load(sb, sd + 48);
     const int oo = 4 * g + kq;
-    const uint32_t hn = (lds_u8(sb, sd + 32 + oo / 2) >> (4 * (oo & 1))) & 15u;
-    const uint32_t qi = lds_u8(sb, sd + oo) | (hn << 8);
+    const uint32_t hb = lds_u8(sb, sd + 32 + oo / 2);
+    const uint32_t ql = lds_u8(sb, sd + oo);
+    after_fields();
+    const uint32_t qi = ql | (((hb >> (4 * (oo & 1))) & 15u) << 8);
+    const uint4 e = *reinterpret_cast<const uint4*>(tbl + qi * 16);
+    const uint32_t wa = ww.get(0), wb = ww.get(1);
+    const uint32_t w0 = wa & 0xFFFFu, w1 = wa >> 16, w2 = wb & 0xFFFFu, w3 = wb >> 16;
+    const uint32_t dbits = ((w0 & 61440u) >> 12) | ((w1 & 61440u) >> 8) | ((w2 & 61440u) >> 4) | (w3 & 61440u);
     const int sci = 2 * g + (kq >> 1);
-    const uint32_t ww = (sci >> 2) == 0 ? w0 : ((sci >> 2) == 1 ? w1 : ((sci >> 2) == 2 ? w2 : w3));
-    const uint32_t sc = (ww >> (3 * (sci & 3))) & 7u;
-    const float d = h2f(dbits) * (float)(2u * sc + 1u);
-    grid8<false>(tbl, qi, d, 0.f, nullptr, o);
+    const uint32_t sw = (sci >> 2) == 0 ? w0 : ((sci >> 2) == 1 ? w1 : ((sci >> 2) == 2 ? w2 : w3));
+    const float d = h2f(dbits) * (float)(2u * ((sw >> (3 * (sci & 3))) & 7u) + 1u);
+    after_lookups();
+    grid8(e, d, o);
   }
 };
+
+#undef GSQ_QMM_RUN
 
 // ---- raw fragments for the small-batch kernel ----------------------------------------------
 // QmsRaw<T>::run gives the eight weights of octet kq of group g without the group's common

@@ -93,18 +93,17 @@ constexpr int qmm_tbl_bytes() {
 }
 
 // LDS plan of (type, activation tile height MF x 16 rows, waves): table image, activation ring
-// of kLx K32 stages (as deep as the LDS left over allows, up to 8), the waves' weight rings and
-// a small broadcast slot.
+// of kLx K32 stages (as deep as the LDS left over allows, up to 8) and the waves' weight rings.
 template <int T, int MF, int WV>
 struct QmmPlan {
   static constexpr int kTbl = qmm_tbl_bytes<T>();
   static constexpr int kW = WV * QmmGeo<T, WV>::kRing;
-  static constexpr int kLx0 = (kQLds - kTbl - kW - 32) / (16 * MF * 64);
-  static constexpr int kLx = kLx0 > 8 ? 8 : kLx0;
+  static constexpr int kLx0 = (kQLds - kTbl - kW) / (16 * MF * 64);
+  // a third stage alone is no gain over two (no barrier saved; IQ1_S at 2048 rows 431 against 414 us)
+  static constexpr int kLx = kLx0 > 8 ? 8 : (kLx0 == 3 ? 2 : kLx0);
   static constexpr int kXOff = kTbl;
   static constexpr int kWOff = kXOff + kLx * 16 * MF * 64;
-  static constexpr int kBcOff = kWOff + kW;
-  static constexpr int kLds = kBcOff + 32;
+  static constexpr int kLds = kWOff + kW;
   static constexpr bool kValid = kLx >= 2 && MF >= WV;  // every wave issues activation DMA
 };
 
@@ -112,8 +111,7 @@ struct QmmPlan {
 // activation stages 0 .. P-1; each stage issues the next activation stage (NX instructions,
 // while it exists) and, at a column start, the next column (GW instructions). With one barrier
 // per stage (BP false), P = LX - 1 and stage q issues activation stage q + LX - 1; it needs the
-// column of stage q + 1 and activation stage q + 1 when the A operands are read one stage
-// ahead (PF), else activation stage q. With one barrier per pair of stages (BP: rings of four
+// column of stage q + 1 and activation stage q. With one barrier per pair of stages (BP: rings of four
 // or more stages), P = LX - 2 and the pair (q, q + 1), q even, issues activation stages
 // q + LX - 2 and q + LX - 1 after its barrier, into the slots of stages q - 2 and q - 1, which
 // every wave has finished; it needs activation stages q and q + 1 and the columns of stages
@@ -144,13 +142,13 @@ constexpr int qmm_end_w(int c, int Q, int LX, int NX, int GW, bool BP) {
   const int nx = BP ? (qp + LX - 2 < Q ? 1 : 0) + (qp + LX - 1 < Q ? 1 : 0) : (qp + LX - 1 < Q ? 1 : 0);
   return qmm_issued_before(qp, Q, LX, NX, GW, BP) + NX * nx + GW;
 }
-constexpr int qmm_wait_n(int q, int Q, int LX, int NX, int GW, bool BP, bool PF) {
+constexpr int qmm_wait_n(int q, int Q, int LX, int NX, int GW, bool BP) {
   int need = 0, wc = -1;
   if (BP) {
     need = qmm_end_x(q + 1, Q, LX, NX, GW, true);
     wc = (q + 2 < Q ? q + 2 : q + 1) >> 3;
   } else {
-    need = qmm_end_x(PF && q + 1 < Q ? q + 1 : q, Q, LX, NX, GW, false);
+    need = qmm_end_x(q, Q, LX, NX, GW, false);
     wc = q + 1 < Q ? (q + 1) >> 3 : -1;
   }
   if (wc >= 0) {
@@ -165,13 +163,13 @@ struct QmmWaitSet {
   int v[64];
   int n;
 };
-template <int LX, int NX, int GW, bool BP, bool PF>
+template <int LX, int NX, int GW, bool BP>
 constexpr QmmWaitSet qmm_wait_set() {
   QmmWaitSet w{};
   w.n = 0;
   for (int cols = 1; cols <= 40; ++cols)
     for (int q = 0; q < 8 * cols; q += BP ? 2 : 1) {
-      int c = qmm_wait_n(q, 8 * cols, LX, NX, GW, BP, PF);
+      int c = qmm_wait_n(q, 8 * cols, LX, NX, GW, BP);
       if (c > 63) c = 63;
       bool seen = false;
       for (int i = 0; i < w.n; ++i) seen = seen || w.v[i] == c;
@@ -192,15 +190,15 @@ __device__ __forceinline__ void wait_vm_imm() {
 }
 // s_waitcnt vmcnt(c) for the largest schedule count c <= n: a short chain of compile-time
 // immediates, largest (steady-state) counts first
-template <int LX, int NX, int GW, bool BP, bool PF, int K = 0>
+template <int LX, int NX, int GW, bool BP, int K = 0>
 __device__ __forceinline__ void qmm_wait(int n) {
-  constexpr QmmWaitSet W = qmm_wait_set<LX, NX, GW, BP, PF>();
+  constexpr QmmWaitSet W = qmm_wait_set<LX, NX, GW, BP>();
   if constexpr (K >= W.n) {
     wait_vm_imm<0>();
   } else {
     constexpr int c = W.v[K];
     if (n >= c) wait_vm_imm<c>();
-    else qmm_wait<LX, NX, GW, BP, PF, K + 1>(n);
+    else qmm_wait<LX, NX, GW, BP, K + 1>(n);
   }
 }
 
@@ -221,25 +219,24 @@ struct QmmMfmaArgs {
   const uint8_t* tbl;    // the type's table image (codebook + sign masks), or null
   int tbl_bytes;         // multiple of 16
   float* part;           // 2 * G partial slots of slot_floats
-  int slot_floats;       // floats per partial slot: MF * NB * 64 * WV * 4 (BM x 256)
+  int slot_floats;       // floats per partial slot: MC * NB * 64 * WV * 4 (a tile)
   long long part_bytes;  // capacity of `part`
-  int* cnt;              // per-tile arrival counters, indexed by the tile's first workgroup
 };
 
-// Partial tiles travel between workgroups (possibly on different XCDs, whose L2 caches are
-// not coherent with each other) as whole 16-byte buffer stores written through to the
-// device-coherent level (sc1) and buffer loads that bypass the caches (sc0 sc1): no L2
-// write-back or invalidate of unrelated data, and full cache lines per wave instruction.
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-// A slot holds one workgroup's partial tile: `slot_floats` floats (the plan's tile size).
+// A partial tile goes to the workspace as whole 16-byte stores in accumulator order (block (i, j)
+// of the thread at ((i NB + j) 64 WV + thread) * 16 bytes of the slot) and is read back the same
+// way by the reduction kernel, so both sides move whole cache lines. Slot 2w: the tile workgroup w
+// starts in; slot 2w + 1: the tile it ends in.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t qmm_slot_rsrc(float* part, int slot, int slot_floats) {
   return __builtin_amdgcn_make_buffer_rsrc(part + (size_t)slot * (size_t)slot_floats, 0, slot_floats * 4, 0x00020000);
 }
-__device__ __forceinline__ void qmm_st_coherent(__amdgpu_buffer_rsrc_t r, int off, float4_t v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, off, 0, 16 /* sc1 */);
-}
-__device__ __forceinline__ float4_t qmm_ld_coherent(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 17 /* sc0 sc1 */));
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+
+// The weight row (0 .. 16 NB - 1 of a wave's rows) decoded as operand row r of its block j: a
+// lane's accumulators of the NB blocks then hold 4 NB consecutive outputs of one activation row.
+template <int NB>
+__device__ __forceinline__ int qmm_row(int j, int r) {
+  return 4 * NB * (r >> 2) + 4 * j + (r & 3);
 }
 
 // workgroup whose range holds column u: ranges are [floor(w*units/G), floor((w+1)*units/G))
@@ -263,78 +260,64 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-template <int MF, int NB>
-__device__ __forceinline__ void qmm_store_tile(void* y, int ydt, int M, int N, const float4_t (&acc)[MF][NB], int m0,
-                                               int n0, int lane) {
-  static_for<MF>([&](auto ic) {
-    constexpr int i = decltype(ic)::value;
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int n = n0 + 16 * j + (lane & 15);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * i + 4 * (lane >> 4) + e;
-        if (m < M && n < N) qmm_store_y(y, ydt, (int64_t)m * N + n, acc[i][j][e]);
-      }
-    }
-  });
-}
-
-// One 16-row block of a wave's output (v[j][e]: row m + 4 (lane / 16) + e, column
-// n0 + 16 j + lane % 16) written as whole row pieces: the wave transposes it through its own
-// LDS area `st` (16 rows of 16 NB floats, row stride 16 NB + 4) and every lane stores 8
-// consecutive fp32 outputs of one row with two 16-byte stores, so each row piece of 64 NB bytes
-// is written whole (the accumulator layout alone gives four rows of 64 bytes per store
-// instruction). The LDS operations of one wave complete in order, so the reads see the writes.
+// The outputs of one 16-row activation block held by a lane (row m + lane % 16; v[j][e]: column
+// n0 + 4 NB (lane / 16) + 4 j + e): 4 NB consecutive ones, stored in whole 16-byte pieces when the
+// rows allow it (vec: y 16-byte aligned and rows of whole 16-byte pieces).
 template <int NB>
-__device__ __forceinline__ void qmm_store_rows_f32(float* y, int M, int N, const float4_t (&v)[NB], int m, int n0,
-                                                   int lane, float* st) {
-  constexpr int W = 16 * NB, S = W + 4, LPR = W / 8, RPP = 64 / LPR;
+__device__ __forceinline__ void qmm_store_block(void* y, int ydt, bool vec, int M, int N, const float4_t (&v)[NB], int m,
+                                                int n0, int lane) {
+  const int mm = m + (lane & 15), n = n0 + 4 * NB * (lane >> 4);
+  if (mm >= M) return;
+  const int64_t at = (int64_t)mm * N + n;
+  if (vec && n + 4 * NB <= N) {
+    if (ydt == QDT_F32) {
 #pragma unroll
-  for (int j = 0; j < NB; ++j)
+      for (int j = 0; j < NB; ++j) __builtin_nontemporal_store(v[j], reinterpret_cast<float4_t*>(static_cast<float*>(y) + at) + j);
+    } else {
+      u32x4_t o[NB / 2];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) st[(4 * (lane >> 4) + e) * S + 16 * j + (lane & 15)] = v[j][e];
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
-  for (int r0 = 0; r0 < 16; r0 += RPP) {
-    const int r = r0 + lane / LPR, c = 8 * (lane % LPR);
-    if (r < 16) {
-      const float4_t a = *reinterpret_cast<const float4_t*>(st + r * S + c);
-      const float4_t b = *reinterpret_cast<const float4_t*>(st + r * S + c + 4);
-      const int mm = m + r, nn = n0 + c;
-      if (mm < M) {
-        float* yp = y + (int64_t)mm * N + nn;
-        if (nn + 8 <= N) {
-          __builtin_nontemporal_store(a, reinterpret_cast<float4_t*>(yp));
-          __builtin_nontemporal_store(b, reinterpret_cast<float4_t*>(yp + 4));
-        } else {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            if (nn + k < N) yp[k] = a[k];
-            if (nn + 4 + k < N) yp[4 + k] = b[k];
+        for (int e = 0; e < 4; e += 2) {
+          uint32_t lo, hi;
+          if (ydt == QDT_F16) {
+            lo = __builtin_bit_cast(uint16_t, (_Float16)v[j][e]);
+            hi = __builtin_bit_cast(uint16_t, (_Float16)v[j][e + 1]);
+          } else {
+            lo = f32_to_bf16_bits(v[j][e]) & 0xFFFFu;
+            hi = f32_to_bf16_bits(v[j][e + 1]) & 0xFFFFu;
           }
+          o[j / 2][2 * (j & 1) + e / 2] = lo | (hi << 16);
         }
-      }
+#pragma unroll
+      for (int j = 0; j < NB / 2; ++j) *(reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(y) + at) + j) = o[j];
     }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + 4 * j + e < N) qmm_store_y(y, ydt, at + 4 * j + e, v[j][e]);
   }
 }
 
 // Issues the activation stages of one workgroup in order: stage q (ring slot b) of tile t,
 // column c; row[i] = this lane's source row (clamped to the matrix) and octet for DMA
 // instruction i, laid out for the XOR-swizzled ring (octet o of row m at o ^ ((m >> 2) & 3)).
-template <int NX, int BM, int LX>
+template <int NX, int BM, int TM, int LX>
 struct QmmXIter {
   const _Float16* x;
   int M, K, mt, nt, nfast, nblk;
   int q, t, c, b;
   const _Float16* row[NX];
   __device__ __forceinline__ void rows(int wave, int lane) {
-    const int m0 = (nfast ? t / nt : t % mt) * BM;
+    const int m0 = (nfast ? t / nt : t % mt) * TM;
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const int s = (wave * NX + i) * 64 + lane;
       const int m = s >> 2;
       const int o = (s & 3) ^ ((m >> 2) & 3);
-      row[i] = x + (long long)min(m0 + m, M - 1) * K + 8 * o;
+      row[i] = x + (long long)min(m0 + min(m, TM - 1), M - 1) * K + 8 * o;
     }
   }
   __device__ __forceinline__ void init(const _Float16* x_, int M_, int K_, int mt_, int nt_, int nfast_, int nblk_, int ub,
@@ -381,7 +364,14 @@ struct QmmTblLds<0> {
   __device__ __forceinline__ static uint8_t* get() { return nullptr; }
 };
 
-template <int T, int MF, bool A4, int WV>
+// Whether a wave's MFMAs are spread over the phases of its decode (see the stage below) or follow
+// it. Spread: 5-9% faster at 512 and 2048 rows of 17408 x 5120 for IQ3_S and IQ3_XXS, 1-7% for the
+// others, except Q6_K and IQ2_S (2048 rows 570 against 541 us and 448 against 434), whose decodes
+// hold more registers and are better scheduled whole.
+template <int T>
+constexpr bool qmm_spread() { return T != Q6_K && T != IQ2_S; }
+
+template <int T, int MF, int MC, bool A4, int WV>
 __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) {
   // the arguments as plain values (no reference to the argument block escapes, so it is never
   // copied to scratch memory, whose loads would wait on the DMA counter)
@@ -397,11 +387,11 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
   const uint8_t* const tblg = args.tbl;
   float* const part = args.part;
   const int slot_floats = args.slot_floats;
-  int* const cnt = args.cnt;
   using Geo = QmmGeo<T, WV>;
   constexpr int BB = Geo::kBB, GW = Geo::kGW, GR = Geo::kGran, S = Geo::kSlot;
   constexpr int RW = Geo::kRows, NB = Geo::kNB, TH = 64 * WV;
   constexpr int BM = 16 * MF, NX = MF / WV;  // NX: activation DMA instructions per wave per stage
+  constexpr int TM = 16 * MC;                // activation rows of a tile (the stage's rows past them repeat the last)
   using Plan = QmmPlan<T, MF, WV>;
   constexpr int LX = Plan::kLx;
   static_assert(Plan::kValid, "activation ring needs two stages");
@@ -426,7 +416,7 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
   if (tbl_bytes) dma_copy(tblg, tbl_bytes, tbl, wave, WV, lane);
 
   // activation stages are issued in order by an iterator
-  QmmXIter<NX, BM, LX> xi;
+  QmmXIter<NX, BM, TM, LX> xi;
   xi.init(xg, M, K, mt, nt, nfast, nblk, ub, wave, lane);
   // weight column cl (local index): the wave's RW superblocks, granule e of the column at
   // byte 16e (row e / GR, granule e % GR of that row); granules past a row's last one reload
@@ -441,7 +431,7 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
     for (int i = 0; i < GW; ++i) {
       const int e = i * 64 + lane;
       const int r = min(e / GR, RW - 1), qg = e - (e / GR) * GR;
-      const int n = min(n0 + r, N - 1);
+      const int n = min(n0 + qmm_row<NB>(r >> 4, r & 15), N - 1);
       const uintptr_t p = reinterpret_cast<uintptr_t>(packed) + (uintptr_t)((long long)n * row_bytes) +
                           (uintptr_t)c * BB;
       const uintptr_t a0 = p & ~(uintptr_t)15;
@@ -451,24 +441,25 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
     }
   };
 
-  // A operands one stage ahead when the ring has a stage to spare: stage q reads stage q + 1's
-  // activations while its MFMAs run on the operands read during stage q - 1
-  constexpr bool PF = LX >= 3 && WV == 4;
   // one barrier per pair of stages when the ring has four or more stages (the DMA schedule
   // above; the waves drift apart by up to a stage between barriers)
-  constexpr bool BP = !PF && LX >= 4;
+  constexpr bool BP = LX >= 4;
   const int P = qmm_pro_x(Q, lx, BP);
 
-  // B operands of stage q: the four 16-row blocks of the wave's weight rows, group q % 8 of
-  // column q / 8; dl = the low address bits of the lane's four superblocks in that column
-  auto decode = [&](int q, const uint32_t (&dl)[NB], half8_t (&bf)[NB]) {
+  // B operands of stage q: the 16-row blocks of the wave's weight rows, group q % 8 of column
+  // q / 8; dl = the low address bits of the lane's superblocks in that column. work(c) (c = 0 ..
+  // 3 NB - 1, compile-time) runs between the phases of the decode.
+  auto decode = [&](int q, const uint32_t (&dl)[NB], half8_t (&bf)[NB], auto work) __attribute__((always_inline)) {
     const uint8_t* wb = wring + ((q >> 3) & 1) * Geo::kCol;
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
+    static_for<NB>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
       uint32_t o[4];
-      QmmDec<T, A4>::run(wb + (16 * j + (lane & 15)) * S, dl[j], tbl, q & 7, lane >> 4, o);
+      QmmDec<T, A4>::run(wb + (16 * j + (lane & 15)) * S, dl[j], tbl, q & 7, lane >> 4, o,
+                         [&] { work(std::integral_constant<int, 3 * j>{}); },
+                         [&] { work(std::integral_constant<int, 3 * j + 1>{}); });
       bf[j] = __builtin_bit_cast(half8_t, o);
-    }
+      work(std::integral_constant<int, 3 * j + 2>{});
+    });
   };
   auto col_delta = [&](int q, uint32_t (&dl)[NB]) {
     const int u = ub + (q >> 3);
@@ -476,41 +467,31 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
     const int n0 = tile_n(tl) * kQBN + wave * RW;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const int n = min(n0 + 16 * j + (lane & 15), N - 1);
+      const int n = min(n0 + qmm_row<NB>(j, lane & 15), N - 1);
       dl[j] = (uint32_t)((reinterpret_cast<uintptr_t>(packed) + (uintptr_t)((long long)n * row_bytes) +
                           (uintptr_t)c * BB) & 15u);
     }
   };
   // A operands of a stage: MF 16-row blocks (row l % 16, octet l / 16, swizzled)
   const int xoff = (lane & 15) * 64 + (((lane >> 4) ^ ((lane >> 2) & 3)) << 4);
-  auto load_a = [&](int slot, half8_t (&af)[MF]) {
-    const uint32_t* xb = reinterpret_cast<const uint32_t*>(xring + slot * (BM * 64) + xoff);
-#pragma unroll
-    for (int i = 0; i < MF; ++i) {
-      const uint32_t* p = xb + i * 256;
-      const uint32_t aw[4] = {p[0], p[1], p[2], p[3]};
-      af[i] = __builtin_bit_cast(half8_t, aw);
-    }
+  auto load_a = [&](int slot, int i) {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(xring + slot * (BM * 64) + xoff) + i * 256;
+    const uint32_t aw[4] = {p[0], p[1], p[2], p[3]};
+    return __builtin_bit_cast(half8_t, aw);
   };
-  int* bc = reinterpret_cast<int*>(dyn + Plan::kBcOff);
-  // the per-wave transpose areas of the final row stores, over the rings
-  constexpr int kSt = 16 * (16 * NB + 4);  // floats per wave
-  static_assert(WV * kSt * 4 <= Plan::kBcOff - Plan::kXOff, "row-store areas exceed the rings");
-  float* const st = reinterpret_cast<float*>(xring) + wave * kSt;
-  const bool yrows = ydt == QDT_F32 && (N & 3) == 0 && (reinterpret_cast<uintptr_t>(yg) & 15) == 0;
+  const bool yvec = (reinterpret_cast<uintptr_t>(yg) & 15) == 0 && (N & (ydt == QDT_F32 ? 3 : 7)) == 0;
 
   // prologue: table, column 0 and the first activation stages in flight; stage 0's weights
   issue_w(0);
   for (int q = 0; q < P; ++q) xi.issue(xring, wave, lane);
-  qmm_wait<LX, NX, GW, BP, PF>(NX * (P - 1));  // table, column 0 and stage 0 (this wave's share)
+  qmm_wait<LX, NX, GW, BP>(NX * (P - 1));  // table, column 0 and stage 0 (this wave's share)
   __syncthreads();
   uint32_t dl[NB];
   col_delta(0, dl);
   half8_t bcur[NB];
-  decode(0, dl, bcur);
-  half8_t acur[MF], anext[MF], bnext[NB];
-  if constexpr (PF) load_a(0, acur);
-  int rb = PF ? 1 : 0;  // ring slot of the next activations read
+  decode(0, dl, bcur, [](auto) {});
+  half8_t bnext[NB];
+  int rb = 0;  // ring slot of the next activations read
 
   // one segment = this workgroup's columns of one tile; stage q multiplies its activations
   // with weights decoded during stage q - 1 and decodes the weights of stage q + 1
@@ -518,23 +499,25 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
     const int u0 = ub + (q0 >> 3);
     const int tile = u0 / nblk;
     const int q1 = q0 + 8 * (min(ue, (tile + 1) * nblk) - u0);
-    const int m0 = tile_m(tile) * BM, n0 = tile_n(tile) * kQBN + wave * RW;
-    float4_t acc[MF][NB];
+    const int m0 = tile_m(tile) * TM, n0 = tile_n(tile) * kQBN + wave * RW;
+    float4_t acc[MC][NB];
 #pragma unroll
-    for (int i = 0; i < MF; ++i)
+    for (int i = 0; i < MC; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
 
-    // stage q: the operands (ua, ub_) were read and decoded during stage q - 1; this stage reads
-    // and decodes those of stage q + 1 into (na, nb). Two stages per iteration with the roles
-    // of the register sets swapped, so no operand is copied between stages.
-    auto stage = [&](int q, const half8_t (&ua)[MF], const half8_t (&ub_)[NB], half8_t (&na)[MF],
-                     half8_t (&nb)[NB]) __attribute__((always_inline)) {
+    // stage q: its weights ub_ were decoded during stage q - 1; this stage decodes those of stage
+    // q + 1 into nb (after the last stage from stale, in-bounds LDS: not used). The MFMAs are
+    // spread over the decode: between its phases (LDS field reads, codebook reads, arithmetic) the
+    // wave issues the MFMAs of a few 16-row activation blocks, whose operands were read AD blocks
+    // ahead, so that no LDS latency is waited for without work to cover it.
+    constexpr int AD = MC < 4 ? MC : 4, NW = 3 * NB;
+    auto stage = [&](int q, const half8_t (&ub_)[NB], half8_t (&nb)[NB]) __attribute__((always_inline)) {
       const int cl = q >> 3;
       if (!BP || (q & 1) == 0) {
         // the activations read until the next wait and the columns decoded until then have
         // landed (this wave's DMAs)
-        qmm_wait<LX, NX, GW, BP, PF>(qmm_wait_n(q, Q, lx, NX, GW, BP, PF));
+        qmm_wait<LX, NX, GW, BP>(qmm_wait_n(q, Q, lx, NX, GW, BP));
         // every wave's DMAs of those stages are in; every wave is done with the slots of the
         // stages before them
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -546,154 +529,111 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
         }
         if ((q & 7) == 0 && cl + 1 < ncols) issue_w(cl + 1);
       }
-      // weights of stage q + 1 (after the last stage they come from stale, in-bounds LDS and
-      // are not used): unconditional, in one scheduling region with the MFMAs
       if (((q + 1) & 7) == 0) col_delta(q + 1, dl);
-      decode(q + 1, dl, nb);
-      // LDS reads stay in this order: the decode's table reads are waited for without waiting
-      // for the activation reads issued after them (LDS completes in order)
-      __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x8);
-      // a wave issuing its MFMAs takes issue priority over the SIMD's other wave, which is
-      // still decoding: the matrix pipe gets its next instruction as soon as it can take one
-      // (2-4% faster at M = 512 and 2048)
-      __builtin_amdgcn_s_setprio(1);
-      // stage q + 1's activations (after the last stage: stale, in-bounds LDS, not used), or
-      // stage q's without the lookahead
-      load_a(rb, na);
+      half8_t a[MC];
+      auto mma = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ub_[j], a[i], acc[i][j], 0, 0, 0);
+      };
+      if constexpr (qmm_spread<T>()) {
+        static_for<AD>([&](auto ic) { a[decltype(ic)::value] = load_a(rb, decltype(ic)::value); });
+        decode(q + 1, dl, nb, [&](auto cc) __attribute__((always_inline)) {
+          constexpr int c = decltype(cc)::value, i0 = c * MC / NW, i1 = (c + 1) * MC / NW;
+          __builtin_amdgcn_sched_barrier(0);
+          static_for<i1 - i0>([&](auto ic) {
+            constexpr int i = i0 + decltype(ic)::value;
+            mma(std::integral_constant<int, i>{});
+            if constexpr (i + AD < MC) a[i + AD] = load_a(rb, i + AD);
+          });
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      } else {
+        decode(q + 1, dl, nb, [](auto) {});
+        // LDS reads stay in this order: the decode's table reads are waited for without waiting
+        // for the activation reads issued after them (LDS completes in order)
+        __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x8);
+        // a wave issuing its MFMAs takes issue priority over the SIMD's other wave, which is
+        // still decoding: the matrix pipe gets its next instruction as soon as it can take one
+        // (2-4% faster at M = 512 and 2048)
+        __builtin_amdgcn_s_setprio(1);
+        static_for<MC>([&](auto ic) { a[decltype(ic)::value] = load_a(rb, decltype(ic)::value); });
+        static_for<MC>(mma);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
+      }
       if (++rb == lx) rb = 0;
-#pragma unroll
-      for (int i = 0; i < MF; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(PF ? ua[i] : na[i], ub_[j], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);  // stages stay apart: two sets of operands at most
-      __builtin_amdgcn_s_setprio(0);
     };
     // a segment is whole columns: its stage count is a multiple of 8
     for (int q = q0; q < q1; q += 2) {
-      stage(q, acur, bcur, anext, bnext);
-      stage(q + 1, anext, bnext, acur, bcur);
+      stage(q, bcur, bnext);
+      stage(q + 1, bnext, bcur);
     }
 
-    // end of this workgroup's part of `tile`
-    const int wf = qmm_owner(tile * nblk, units, G);
-    const int wl = qmm_owner(tile * nblk + nblk - 1, units, G);
-    // after the workgroup's last stage the rings hold nothing that is still needed: fp32 rows
-    // of the tile are then written whole through a per-wave LDS transpose
-    const bool end_lds = yrows && q1 == Q;
-    // direct: this workgroup's accumulators hold the whole tile (its only piece, or the other
-    // pieces' partials added in place below)
-    constexpr int CH = 8;  // output blocks per batch of partial loads
-    bool direct = wf == wl;
-    bool last = false;
-    if (!direct) {
-      // slot 2w: the tile this workgroup starts in; slot 2w + 1: the tile it ends in
-      const int slot = 2 * w + (q0 == 0 ? 0 : 1);
-      // the workgroup holding the tile's first columns (its range's last work, so often the
-      // last to arrive) looks at the arrival count first: if every other piece is in, it stores
-      // no partial and adds the others' partials to its accumulators in place, in workgroup
-      // order from +0, the same sums as the memory path below (it also takes this path when
-      // its own increment shows it last)
-      const bool own = w == wf;
-      if (tid == 0) bc[0] = own ? __hip_atomic_load(&cnt[wf], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
-      __syncthreads();
-      last = bc[0] == wl - wf;
-      if (!last) {
-        const __amdgpu_buffer_rsrc_t ps = qmm_slot_rsrc(part, slot, slot_floats);
-        // every store has completed (device-coherent) before the arrival count is incremented;
-        // 16-row blocks wholly past M (padding rows of the last activation tile) are not stored
-#pragma unroll
-        for (int i = 0; i < MF; ++i)
-          if (m0 + 16 * i < M) {
-#pragma unroll
-            for (int j = 0; j < NB; ++j) qmm_st_coherent(ps, ((i * NB + j) * TH + tid) * 16, acc[i][j]);
-          }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (tid == 0) bc[1] = __hip_atomic_fetch_add(&cnt[wf], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        last = bc[1] == wl - wf;
-      }
-      if (last && own) {
-#pragma unroll
-        for (int i = 0; i < MF; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f} + acc[i][j];
-        for (int v = wf + 1; v <= wl; ++v) {
-          const int vs = 2 * v + (tile == qmm_first_col(v, units, G) / nblk ? 0 : 1);
-          const __amdgpu_buffer_rsrc_t pv = qmm_slot_rsrc(part, vs, slot_floats);
-#pragma unroll
-          for (int ij0 = 0; ij0 < MF * NB; ij0 += CH) {
-            if (m0 + 16 * (ij0 / NB) < M) {
-              float4_t ld[CH];
-#pragma unroll
-              for (int t = 0; t < CH; ++t) ld[t] = qmm_ld_coherent(pv, ((ij0 + t) * TH + tid) * 16);
-#pragma unroll
-              for (int t = 0; t < CH; ++t) acc[(ij0 + t) / NB][(ij0 + t) % NB] += ld[t];
-            }
-          }
-        }
-        if (tid == 0) __hip_atomic_store(&cnt[wf], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        direct = true;
-      }
-    }
-    if (direct) {
-      if (end_lds) {
-        __syncthreads();  // every wave is done with the rings
-        static_for<MF>([&](auto ic) {
-          constexpr int i = decltype(ic)::value;
-          if (m0 + 16 * i < M) qmm_store_rows_f32<NB>(static_cast<float*>(yg), M, N, acc[i], m0 + 16 * i, n0, lane, st);
-        });
-      } else {
-        qmm_store_tile<MF, NB>(yg, ydt, M, N, acc, m0, n0, lane);
-      }
+    // end of this workgroup's part of `tile`: the whole tile goes to y, a part of it to the
+    // workspace, summed by the reduction kernel; 16-row blocks wholly past M go nowhere
+    const bool whole = u0 == tile * nblk && q1 - q0 == 8 * nblk;
+    if (whole) {
+      static_for<MC>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if (m0 + 16 * i < M) qmm_store_block<NB>(yg, ydt, yvec, M, N, acc[i], m0 + 16 * i, n0, lane);
+      });
     } else {
-      if (last) {  // sum the partials in workgroup order
-        const int mb = m0 + 4 * (lane >> 4), nb = n0 + (lane & 15);
-#pragma unroll 1
-        for (int ij0 = 0; ij0 < MF * NB; ij0 += CH) {
-          // batches that start past M hold only padding rows, whose partials were not stored
-          if (m0 + 16 * (ij0 / NB) >= M) break;
-          float4_t sum[CH];
+      const __amdgpu_buffer_rsrc_t ps = qmm_slot_rsrc(part, 2 * w + (q0 == 0 ? 0 : 1), slot_floats);
+      static_for<MC>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if (m0 + 16 * i < M) {
 #pragma unroll
-          for (int t = 0; t < CH; ++t) sum[t] = (float4_t){0.f, 0.f, 0.f, 0.f};
-          for (int v = wf; v <= wl; ++v) {
-            const int vs = 2 * v + (tile == qmm_first_col(v, units, G) / nblk ? 0 : 1);
-            const __amdgpu_buffer_rsrc_t pv = qmm_slot_rsrc(part, vs, slot_floats);
-            float4_t ld[CH];
-#pragma unroll
-            for (int t = 0; t < CH; ++t) ld[t] = qmm_ld_coherent(pv, ((ij0 + t) * TH + tid) * 16);
-#pragma unroll
-            for (int t = 0; t < CH; ++t) sum[t] += ld[t];
-          }
-          if (end_lds) {
-#pragma unroll
-            for (int a = 0; a < CH / NB; ++a) {
-              const int i = ij0 / NB + a;
-              float4_t v[NB];
-#pragma unroll
-              for (int j = 0; j < NB; ++j) v[j] = sum[a * NB + j];
-              if (m0 + 16 * i < M) qmm_store_rows_f32<NB>(static_cast<float*>(yg), M, N, v, m0 + 16 * i, n0, lane, st);
-            }
-          } else {
-#pragma unroll
-            for (int t = 0; t < CH; ++t) {
-              const int ij = ij0 + t;
-              const int n = nb + 16 * (ij % NB);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const int m = mb + 16 * (ij / NB) + e;
-                if (m < M && n < N) qmm_store_y(yg, ydt, (int64_t)m * N + n, sum[t][e]);
-              }
-            }
-          }
+          for (int j = 0; j < NB; ++j)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[i][j]), ps, ((i * NB + j) * TH + tid) * 16, 0,
+                                                   16 /* sc1: written through */);
         }
-        if (tid == 0) __hip_atomic_store(&cnt[wf], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      __syncthreads();
+      });
     }
     q0 = q1;
   }
+}
+
+// Sums the partials of the split tiles in workgroup order (deterministic) and writes y: one
+// workgroup per (boundary between two workgroups' ranges, 16-row activation block), working only at
+// the first boundary inside each split tile. Its own launch, so that every CU reads partials at
+// once: summed inside the main kernel by a tile's last workgroup to arrive, one CU read all of a
+// tile's partials (2 to 13 of 128-256 KB) with the others idle, 25-38 us at the end of a launch.
+template <int MC, int NB, int WV>
+__global__ void __launch_bounds__(64 * WV) qmm_reduce_kernel(QmmMfmaArgs a) {
+  constexpr int TH = 64 * WV, UN = 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = blockIdx.y;
+  const int w = (int)blockIdx.x + 1, ub = qmm_first_col(w, a.units, a.G), tile = ub / a.nblk;
+  if (ub == tile * a.nblk || qmm_first_col(w - 1, a.units, a.G) > tile * a.nblk) return;
+  const int m0 = (a.nfast ? tile / a.nt : tile % a.mt) * 16 * MC + 16 * i;
+  if (m0 >= a.M) return;
+  const int n0 = (a.nfast ? tile % a.nt : tile / a.mt) * kQBN + wave * (16 * NB);
+  const int wf = w - 1, wl = qmm_owner(tile * a.nblk + a.nblk - 1, a.units, a.G);
+  // only the first piece can be its workgroup's last work and not its first
+  const int s0 = 2 * wf + (qmm_first_col(wf, a.units, a.G) / a.nblk == tile ? 0 : 1);
+  auto slot = [&](int v) {
+    return a.part + (size_t)(v == wf ? s0 : 2 * v) * (size_t)a.slot_floats + ((size_t)(i * NB) * TH + tid) * 4;
+  };
+  float4_t sum[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) sum[j] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  for (int v = wf; v <= wl; v += UN) {
+    float4_t ld[UN][NB];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {  // clamped to the last piece: its repeats are not added
+      const float* p = slot(v + u <= wl ? v + u : wl);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) ld[u][j] = *reinterpret_cast<const float4_t*>(p + (size_t)j * TH * 4);
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+      if (v + u <= wl) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) sum[j] += ld[u][j];
+      }
+  }
+  const bool vec = (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && (a.N & (a.y_dtype == QDT_F32 ? 3 : 7)) == 0;
+  qmm_store_block<NB>(a.y, a.y_dtype, vec, a.M, a.N, sum, m0, n0, lane);
 }
 
 // ---- generic kernel (fp32 / bf16 activations) ------------------------------------------
@@ -802,6 +742,12 @@ __global__ void __launch_bounds__(256) qmm_generic_kernel(QmmArgs a) {
 
 namespace gsq {
 
+// Tiles of 192 rows where they cover M with fewer 16-row blocks than tiles of 256 (equal: 256, which
+// decode the weights less often).
+static int qmm_tall_blocks(long long M) {
+  return (M + 191) / 192 * 12 < (M + 255) / 256 * 16 ? 12 : 16;
+}
+
 // ---- host side --------------------------------------------------------------------------
 extern QmmTuning g_qmm_tuning;
 
@@ -810,79 +756,54 @@ static bool qmm_grid_type(int qt) {
   return qt == IQ1_S || qt == IQ1_M || qt == IQ2_XXS || qt == IQ2_XS || qt == IQ2_S || qt == IQ3_XXS || qt == IQ3_S;
 }
 
-// Floats of one partial slot of the tiled kernel: every lane of the WV waves stores MF x NB
-// float4 accumulators (a BM x 256 tile).
-template <int T, int MF, int WV>
-constexpr int qmm_slot_floats() { return MF * QmmGeo<T, WV>::kNB * 64 * WV * 4; }
-
-template <int T, int MF, bool A4, int WV>
-static hipError_t launch_mfma_t(QmmMfmaArgs a, hipStream_t s) {
-  if constexpr (!QmmPlan<T, MF, WV>::kValid) {
-    return hipErrorInvalidValue;
-  } else {
-    a.slot_floats = qmm_slot_floats<T, MF, WV>();
-    if (2ll * a.G * a.slot_floats * 4 > a.part_bytes) return hipErrorInvalidValue;
-    auto k = qmm_mfma_kernel<T, MF, A4, WV>;
+// Launch plans of the tiled kernel: ring height MF and tile height MC (16-row blocks) and waves.
+// MF 16 holds tiles of 16 or 12 blocks (192 rows), so that 129-192 rows (and the like of larger
+// batches) do not multiply padding.
+template <int T, int MF, int MC, int WV>
+static hipError_t launch_mfma_t(QmmMfmaArgs a, bool a4, hipStream_t s) {
+  using Plan = QmmPlan<T, MF, WV>;
+  static_assert(Plan::kValid);
+  constexpr int NB = QmmGeo<T, WV>::kNB;
+  constexpr size_t lds = Plan::kLds - Plan::kTbl;  // dynamic part
+  auto go = [&](auto k) -> hipError_t {
     static bool attr_set = false;
     if (!attr_set) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         kQLds - QmmPlan<T, MF, WV>::kTbl);
+      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kQLds - Plan::kTbl);
       if (e != hipSuccess) return e;
       attr_set = true;
     }
-    constexpr size_t lds = QmmPlan<T, MF, WV>::kLds - QmmPlan<T, MF, WV>::kTbl;  // dynamic part
     hipLaunchKernelGGL(k, dim3(a.G), dim3(64 * WV), lds, s, a);
     return hipGetLastError();
-  }
-}
-
-template <int T, int MF, int WV>
-static hipError_t launch_mfma_a4(const QmmMfmaArgs& a, bool a4, hipStream_t s) {
-  if constexpr (BlockBytes<T>::v % 4 == 0) {
-    if (a4) return launch_mfma_t<T, MF, true, WV>(a, s);
-  }
-  return launch_mfma_t<T, MF, false, WV>(a, s);
-}
-// 8 waves where the tile allows it (and the tuning does not ask for 4), else 4
-template <int T, int MF>
-static hipError_t launch_mfma_mf(const QmmMfmaArgs& a, bool a4, bool w8, hipStream_t s) {
-  if constexpr (QmmPlan<T, MF, 8>::kValid) {
-    if (w8) return launch_mfma_a4<T, MF, 8>(a, a4, s);
-  }
-  return launch_mfma_a4<T, MF, 4>(a, a4, s);
-}
-
-// Plan and launch the MFMA kernel for type T: activation tile height (MF 16-row blocks) from M
-// (64 rows up to 64, 128 up to 128, else 256), then the stream-K grid:
-// one workgroup per CU, at most one per (tile, K column) unit.
-// Bytes of one partial slot of the plan launch_mfma_mf<T, mf> picks (8 waves where valid).
-template <int T>
-static long long qmm_slot_bytes(int mf, bool w8) {
-  auto pick = [&](auto mfc) -> long long {
-    constexpr int MF = decltype(mfc)::value;
-    if constexpr (QmmPlan<T, MF, 8>::kValid) {
-      if (w8) return 4ll * qmm_slot_floats<T, MF, 8>();
-    }
-    return 4ll * qmm_slot_floats<T, MF, 4>();
   };
-  if (mf == 4) return pick(std::integral_constant<int, 4>{});
-  if (mf == 8) return pick(std::integral_constant<int, 8>{});
-  return pick(std::integral_constant<int, 16>{});
+  hipError_t e;
+  if constexpr (BlockBytes<T>::v % 4 == 0) {
+    e = a4 ? go(qmm_mfma_kernel<T, MF, MC, true, WV>) : go(qmm_mfma_kernel<T, MF, MC, false, WV>);
+  } else {
+    e = go(qmm_mfma_kernel<T, MF, MC, false, WV>);
+  }
+  // split tiles: unless every workgroup's range starts at a tile's first column
+  if (e == hipSuccess && a.G > 1 && ((long long)a.units % a.G != 0 || (a.units / a.G) % a.nblk != 0)) {
+    hipLaunchKernelGGL((qmm_reduce_kernel<MC, NB, WV>), dim3(a.G - 1, MC), dim3(64 * WV), 0, s, a);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
+// Plan and launch the MFMA kernel for type T: tile height from M (64 rows up to 64, 128 up to 128,
+// 192 or 256 beyond), then the stream-K grid: one workgroup per CU, at most one per two (tile, K
+// column) units.
 template <int T>
 static hipError_t launch_mfma(QmmMfmaArgs& a, int num_cus, const QmmWorkspace& ws, hipStream_t s) {
   if (a.tbl_bytes != qmm_tbl_bytes<T>()) return hipErrorInvalidValue;
-  int mf = g_qmm_tuning.mf;
-  if (mf == 0) mf = a.M <= 64 ? 4 : (a.M <= 128 ? 8 : 16);
-  if (mf != 4 && mf != 8 && mf != 16) return hipErrorInvalidValue;
+  int mc = g_qmm_tuning.mf;
+  if (mc == 0) mc = a.M <= 64 ? 4 : (a.M <= 128 ? 8 : qmm_tall_blocks(a.M));
+  if (mc != 4 && mc != 8 && mc != 12 && mc != 16) return hipErrorInvalidValue;
   const bool a4 = (reinterpret_cast<uintptr_t>(a.packed) & 3) == 0;
-  const bool w8 = g_qmm_tuning.waves != 4;
   // at least min_cols columns per workgroup: fewer workgroups share each tile when the
   // problem is small, which bounds the partial-tile traffic
   const int min_cols = g_qmm_tuning.min_cols > 0 ? g_qmm_tuning.min_cols : 2;
   for (;;) {
-    const int bm = 16 * mf;
+    const int bm = 16 * mc;
     a.mt = (a.M + bm - 1) / bm;
     a.nt = (int)((a.N + kQBN - 1) / kQBN);
     // weight tile fastest: the workgroups of one XCD (consecutive units) share an activation
@@ -895,18 +816,19 @@ static hipError_t launch_mfma(QmmMfmaArgs& a, int num_cus, const QmmWorkspace& w
     a.G = num_cus < gmax ? num_cus : gmax;
     if (a.G > ws.max_groups) a.G = ws.max_groups;
     // a workspace too small for this tile height's partials at this grid: lower tiles
-    if (2ll * a.G * qmm_slot_bytes<T>(mf, w8) <= ws.part_bytes) break;
-    if (mf == 4) return hipErrorInvalidValue;
-    mf /= 2;
+    a.slot_floats = mc * 16 * kQBN;
+    if (2ll * a.G * a.slot_floats * 4 <= ws.part_bytes) break;
+    if (mc == 4) return hipErrorInvalidValue;
+    mc = mc > 8 ? 8 : 4;
   }
   a.xcd_remap = (a.G % 8 == 0) ? 1 : 0;
   a.part = ws.part;
   a.part_bytes = ws.part_bytes;
-  a.cnt = ws.cnt;
-  switch (mf) {
-    case 4: return launch_mfma_mf<T, 4>(a, a4, w8, s);
-    case 8: return launch_mfma_mf<T, 8>(a, a4, w8, s);
-    default: return launch_mfma_mf<T, 16>(a, a4, w8, s);
+  switch (mc) {
+    case 4: return launch_mfma_t<T, 4, 4, 4>(a, a4, s);
+    case 8: return launch_mfma_t<T, 8, 8, 8>(a, a4, s);
+    case 12: return launch_mfma_t<T, 16, 12, 8>(a, a4, s);
+    default: return launch_mfma_t<T, 16, 16, 8>(a, a4, s);
   }
 }
 

@@ -25,10 +25,21 @@
 //    its own groups in A and B alike, with the groups' sub-scales inside the fp16 values and the
 //    superblock's d on the MFMA sum);
 //  * a row group split between workgroups is finished by the last to arrive, which sums
-//    the fp32 partials in workgroup order (deterministic), as in the tiled kernel.
+//    the fp32 partials in workgroup order (deterministic).
 #pragma once
 
 namespace gsq {
+
+// The partials of a row group travel between workgroups of one launch (possibly on different XCDs,
+// whose L2 caches are not coherent with each other) as whole 16-byte buffer stores written
+// through to the device-coherent level (sc1) and buffer loads that bypass the caches (sc0 sc1):
+// no L2 write-back or invalidate of unrelated data, and full cache lines per wave instruction.
+__device__ __forceinline__ void qmm_st_coherent(__amdgpu_buffer_rsrc_t r, int off, float4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, off, 0, 16 /* sc1 */);
+}
+__device__ __forceinline__ float4_t qmm_ld_coherent(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 17 /* sc0 sc1 */));
+}
 
 template <int T, int WV, int NB>
 struct QmsGeo {
