@@ -21,15 +21,14 @@
 //  * all DMA waits are exact s_waitcnt vmcnt counts derived from the fixed issue order; one
 //    s_barrier per K32 stage (per pair of stages on rings of four or more stages) guards the
 //    shared activation ring.
-//  * stream-K work split: the (tile, K column) iterations are divided evenly over as many
-//    workgroups as there are CUs, so shapes whose tile count is not a multiple of the CU count
-//    (17408 = 17 * 1024 rows) still fill the chip. A tile split between workgroups is
-//    finished by the last one to arrive (per-tile arrival counter), which sums the fp32
-//    partials in a fixed order (deterministic) and writes y; the workgroup holding a tile's
-//    first columns keeps its own piece in registers when it finds the others already in.
-//  * tiles are numbered weight tile fastest and workgroups renumbered so that consecutive work
-//    (one activation tile, neighbouring weight tiles and K ranges) lands on one XCD and shares
-//    its L2.
+//  * work split: as many workgroups as there are CUs; each takes whole tiles while there are
+//    enough for all, and the (tile, K column) units of the tiles left over are divided evenly
+//    (stream-K), so shapes whose tile count is not a multiple of the CU count (17408 = 17 * 1024
+//    rows) still fill the chip. Tiles split between workgroups go to a workspace as fp32 partials,
+//    which a second launch sums in a fixed order (deterministic).
+//  * tiles are numbered weight tile fastest and workgroups renumbered so that work done at the
+//    same time (one activation tile, neighbouring weight tiles and K ranges) lands on one XCD and
+//    shares its L2.
 // fp32 / bf16 activations use the generic kernel below.
 #pragma once
 #include <cstdlib>
@@ -213,8 +212,10 @@ struct QmmMfmaArgs {
   int mt;                // activation tiles
   int nt;                // weight tiles (kQBN rows)
   int nfast;             // tile t = (activation tile t / nt, weight tile t % nt), else (t % mt, t / mt)
-  int units;             // tiles * nblk
   int G;                 // workgroups
+  int rounds;            // whole tiles of every workgroup: tile r * G + w in round r
+  int units;             // (tile, K column) units of the tiles after those,
+  int GS;                // split evenly over the first GS workgroups
   int xcd_remap;         // G is a multiple of 8
   const uint8_t* tbl;    // the type's table image (codebook + sign masks), or null
   int tbl_bytes;         // multiple of 16
@@ -261,18 +262,22 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // The outputs of one 16-row activation block held by a lane (row m + lane % 16; v[j][e]: column
-// n0 + 4 NB (lane / 16) + 4 j + e): 4 NB consecutive ones, stored in whole 16-byte pieces when the
-// rows allow it (vec: y 16-byte aligned and rows of whole 16-byte pieces).
+// n0 + 4 NB (lane / 16) + 4 j + e): 4 NB consecutive ones, in 16-byte pieces. Rows of odd N leave
+// the pieces unaligned, which gfx950 stores as well: value by value they cost 31% of a 1227 x 7959
+// x 512 product.
 template <int NB>
-__device__ __forceinline__ void qmm_store_block(void* y, int ydt, bool vec, int M, int N, const float4_t (&v)[NB], int m,
-                                                int n0, int lane) {
+__device__ __forceinline__ void qmm_store_block(void* y, int ydt, int M, int N, const float4_t (&v)[NB], int m, int n0,
+                                                int lane) {
+  typedef float4_t float4u_t __attribute__((aligned(4)));
+  typedef u32x4_t u32x4u_t __attribute__((aligned(2)));
   const int mm = m + (lane & 15), n = n0 + 4 * NB * (lane >> 4);
   if (mm >= M) return;
   const int64_t at = (int64_t)mm * N + n;
-  if (vec && n + 4 * NB <= N) {
+  if (n + 4 * NB <= N) {
     if (ydt == QDT_F32) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) __builtin_nontemporal_store(v[j], reinterpret_cast<float4_t*>(static_cast<float*>(y) + at) + j);
+      for (int j = 0; j < NB; ++j)
+        __builtin_nontemporal_store(v[j], reinterpret_cast<float4u_t*>(static_cast<float*>(y) + at + 4 * j));
     } else {
       u32x4_t o[NB / 2];
 #pragma unroll
@@ -290,7 +295,7 @@ __device__ __forceinline__ void qmm_store_block(void* y, int ydt, bool vec, int 
           o[j / 2][2 * (j & 1) + e / 2] = lo | (hi << 16);
         }
 #pragma unroll
-      for (int j = 0; j < NB / 2; ++j) *(reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(y) + at) + j) = o[j];
+      for (int j = 0; j < NB / 2; ++j) *reinterpret_cast<u32x4u_t*>(static_cast<uint16_t*>(y) + at + 8 * j) = o[j];
     }
   } else {
 #pragma unroll
@@ -307,7 +312,7 @@ __device__ __forceinline__ void qmm_store_block(void* y, int ydt, bool vec, int 
 template <int NX, int BM, int TM, int LX>
 struct QmmXIter {
   const _Float16* x;
-  int M, K, mt, nt, nfast, nblk;
+  int M, K, mt, nt, nfast, nblk, G, c0, left, n, ts, cs;  // left: whole tiles to go, n: columns to go in this one
   int q, t, c, b;
   const _Float16* row[NX];
   __device__ __forceinline__ void rows(int wave, int lane) {
@@ -320,8 +325,9 @@ struct QmmXIter {
       row[i] = x + (long long)min(m0 + min(m, TM - 1), M - 1) * K + 8 * o;
     }
   }
-  __device__ __forceinline__ void init(const _Float16* x_, int M_, int K_, int mt_, int nt_, int nfast_, int nblk_, int ub,
-                                       int wave, int lane) {
+  // `rounds` whole tiles w, w + G, ..., each from column c0 on, then the units from us on
+  __device__ __forceinline__ void init(const _Float16* x_, int M_, int K_, int mt_, int nt_, int nfast_, int nblk_, int G_,
+                                       int rounds, int w, int c0_, int us, int wave, int lane) {
     x = x_;
     M = M_;
     K = K_;
@@ -329,10 +335,16 @@ struct QmmXIter {
     nt = nt_;
     nfast = nfast_;
     nblk = nblk_;
+    G = G_;
+    left = rounds;
+    n = nblk;
+    c0 = c0_;
+    ts = us / nblk;
+    cs = us - ts * nblk;
     q = 0;
     b = 0;
-    t = ub / nblk;
-    c = ub - t * nblk;
+    t = rounds ? w : ts;
+    c = rounds ? c0 : cs;
     rows(wave, lane);
   }
   __device__ __forceinline__ void issue(uint8_t* xring, int wave, int lane) {
@@ -343,10 +355,21 @@ struct QmmXIter {
       __builtin_amdgcn_global_load_lds(static_cast<const void*>(row[i] + kk), (lds_ptr_t)(buf + i * 1024), 16, 0, 0);
     ++q;
     if (++b == LX) b = 0;
-    if ((q & 7) == 0 && ++c == nblk) {
-      c = 0;
-      ++t;
-      rows(wave, lane);
+    if ((q & 7) == 0) {
+      if (++c == nblk) {
+        c = 0;
+        if (left == 0) {
+          ++t;
+          rows(wave, lane);
+        }
+      }
+      if (left > 0 && --n == 0) {
+        --left;
+        n = nblk;
+        t = left ? t + G : ts;
+        c = left ? c0 : cs;
+        rows(wave, lane);
+      }
     }
   }
 };
@@ -382,7 +405,7 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
   const int nt = args.nt, nfast = args.nfast;
   auto tile_m = [&](int t) { return nfast ? t / nt : t % mt; };
   auto tile_n = [&](int t) { return nfast ? t % nt : t / mt; };
-  const int units = args.units, G = args.G, xcd = args.xcd_remap, tbl_bytes = args.tbl_bytes;
+  const int G = args.G, xcd = args.xcd_remap, tbl_bytes = args.tbl_bytes;
   const long long row_bytes = args.row_bytes;
   const uint8_t* const tblg = args.tbl;
   float* const part = args.part;
@@ -400,9 +423,21 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int bid = blockIdx.x;
   const int w = xcd ? (bid & 7) * (G >> 3) + (bid >> 3) : bid;
-  const int ub = qmm_first_col(w, units, G), ue = qmm_first_col(w + 1, units, G);
-  const int ncols = ue - ub;  // >= 1: G <= units
+  // local columns: those of `rounds` whole tiles, then a range of the split units
+  const int rounds = args.rounds, wc = rounds * nblk, split0 = rounds * G * nblk;
+  const int ub = split0 + (w < args.GS ? qmm_first_col(w, args.units, args.GS) : 0);
+  const int ncols = wc + (w < args.GS ? split0 + qmm_first_col(w + 1, args.units, args.GS) - ub : 0);  // >= 1
   const int Q = 8 * ncols;    // K32 stages of this workgroup
+  // whole tiles start at a column of the workgroup's own and wrap around: the 32 workgroups of an
+  // XCD read one activation tile, so each loads a share of it early for the others; all starting
+  // at column 0, every one waited for each column's first read from HBM (2048 rows of 17408 x 5120
+  // IQ3_S with new activations every call 487 -> 459 us)
+  const int c0 = (w & 31) * nblk >> 5;
+  auto unit = [&](int cl) {   // (tile, column) unit of local column cl
+    if (cl >= wc) return ub + cl - wc;
+    const int r = cl / nblk, c = cl - r * nblk + c0;
+    return (r * G + w) * nblk + (c < nblk ? c : c - nblk);
+  };
   constexpr int lx = LX;
   // the table image is static LDS at address 0 (its reads fold the base into their address
   // arithmetic); the plan's other offsets count from the table's start, where dynamic LDS
@@ -417,13 +452,13 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
 
   // activation stages are issued in order by an iterator
   QmmXIter<NX, BM, TM, LX> xi;
-  xi.init(xg, M, K, mt, nt, nfast, nblk, ub, wave, lane);
+  xi.init(xg, M, K, mt, nt, nfast, nblk, G, rounds, w, c0, ub, wave, lane);
   // weight column cl (local index): the wave's RW superblocks, granule e of the column at
   // byte 16e (row e / GR, granule e % GR of that row); granules past a row's last one reload
   // its last granule, and lanes past the last row (whole instructions) reload the last row's,
   // so every lane stays active and the count stays fixed
   auto issue_w = [&](int cl) {
-    const int u = ub + cl;
+    const int u = unit(cl);
     const int tile = u / nblk, c = u - tile * nblk;
     const int n0 = tile_n(tile) * kQBN + wave * RW;
     uint8_t* buf = wring + (cl & 1) * Geo::kCol;
@@ -462,7 +497,7 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
     });
   };
   auto col_delta = [&](int q, uint32_t (&dl)[NB]) {
-    const int u = ub + (q >> 3);
+    const int u = unit(q >> 3);
     const int tl = u / nblk, c = u - tl * nblk;
     const int n0 = tile_n(tl) * kQBN + wave * RW;
 #pragma unroll
@@ -479,8 +514,6 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
     const uint32_t aw[4] = {p[0], p[1], p[2], p[3]};
     return __builtin_bit_cast(half8_t, aw);
   };
-  const bool yvec = (reinterpret_cast<uintptr_t>(yg) & 15) == 0 && (N & (ydt == QDT_F32 ? 3 : 7)) == 0;
-
   // prologue: table, column 0 and the first activation stages in flight; stage 0's weights
   issue_w(0);
   for (int q = 0; q < P; ++q) xi.issue(xring, wave, lane);
@@ -496,9 +529,10 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
   // one segment = this workgroup's columns of one tile; stage q multiplies its activations
   // with weights decoded during stage q - 1 and decodes the weights of stage q + 1
   for (int q0 = 0; q0 < Q;) {
-    const int u0 = ub + (q0 >> 3);
+    const int u0 = unit(q0 >> 3);
     const int tile = u0 / nblk;
-    const int q1 = q0 + 8 * (min(ue, (tile + 1) * nblk) - u0);
+    const bool round = q0 < 8 * wc;
+    const int q1 = q0 + 8 * (round ? nblk : min(ncols - (q0 >> 3), (tile + 1) * nblk - u0));
     const int m0 = tile_m(tile) * TM, n0 = tile_n(tile) * kQBN + wave * RW;
     float4_t acc[MC][NB];
 #pragma unroll
@@ -572,14 +606,14 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
 
     // end of this workgroup's part of `tile`: the whole tile goes to y, a part of it to the
     // workspace, summed by the reduction kernel; 16-row blocks wholly past M go nowhere
-    const bool whole = u0 == tile * nblk && q1 - q0 == 8 * nblk;
+    const bool whole = round || (u0 == tile * nblk && q1 - q0 == 8 * nblk);
     if (whole) {
       static_for<MC>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        if (m0 + 16 * i < M) qmm_store_block<NB>(yg, ydt, yvec, M, N, acc[i], m0 + 16 * i, n0, lane);
+        if (m0 + 16 * i < M) qmm_store_block<NB>(yg, ydt, M, N, acc[i], m0 + 16 * i, n0, lane);
       });
     } else {
-      const __amdgpu_buffer_rsrc_t ps = qmm_slot_rsrc(part, 2 * w + (q0 == 0 ? 0 : 1), slot_floats);
+      const __amdgpu_buffer_rsrc_t ps = qmm_slot_rsrc(part, 2 * w + (u0 == ub ? 0 : 1), slot_floats);
       static_for<MC>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         if (m0 + 16 * i < M) {
@@ -599,18 +633,19 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
 // the first boundary inside each split tile. Its own launch, so that every CU reads partials at
 // once: summed inside the main kernel by a tile's last workgroup to arrive, one CU read all of a
 // tile's partials (2 to 13 of 128-256 KB) with the others idle, 25-38 us at the end of a launch.
-template <int MC, int NB, int WV>
+template <int T, int MC, int NB, int WV>  // T: one kernel symbol per translation unit
 __global__ void __launch_bounds__(64 * WV) qmm_reduce_kernel(QmmMfmaArgs a) {
   constexpr int TH = 64 * WV, UN = 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = blockIdx.y;
-  const int w = (int)blockIdx.x + 1, ub = qmm_first_col(w, a.units, a.G), tile = ub / a.nblk;
-  if (ub == tile * a.nblk || qmm_first_col(w - 1, a.units, a.G) > tile * a.nblk) return;
+  const int w = (int)blockIdx.x + 1, ub = qmm_first_col(w, a.units, a.GS), st = ub / a.nblk;  // st: split tile
+  if (ub == st * a.nblk || qmm_first_col(w - 1, a.units, a.GS) > st * a.nblk) return;
+  const int tile = a.rounds * a.G + st;
   const int m0 = (a.nfast ? tile / a.nt : tile % a.mt) * 16 * MC + 16 * i;
   if (m0 >= a.M) return;
   const int n0 = (a.nfast ? tile % a.nt : tile / a.mt) * kQBN + wave * (16 * NB);
-  const int wf = w - 1, wl = qmm_owner(tile * a.nblk + a.nblk - 1, a.units, a.G);
-  // only the first piece can be its workgroup's last work and not its first
-  const int s0 = 2 * wf + (qmm_first_col(wf, a.units, a.G) / a.nblk == tile ? 0 : 1);
+  const int wf = w - 1, wl = qmm_owner(st * a.nblk + a.nblk - 1, a.units, a.GS);
+  // only the first piece can follow another one in its workgroup's range
+  const int s0 = 2 * wf + (qmm_first_col(wf, a.units, a.GS) / a.nblk == st ? 0 : 1);
   auto slot = [&](int v) {
     return a.part + (size_t)(v == wf ? s0 : 2 * v) * (size_t)a.slot_floats + ((size_t)(i * NB) * TH + tid) * 4;
   };
@@ -632,8 +667,7 @@ __global__ void __launch_bounds__(64 * WV) qmm_reduce_kernel(QmmMfmaArgs a) {
         for (int j = 0; j < NB; ++j) sum[j] += ld[u][j];
       }
   }
-  const bool vec = (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && (a.N & (a.y_dtype == QDT_F32 ? 3 : 7)) == 0;
-  qmm_store_block<NB>(a.y, a.y_dtype, vec, a.M, a.N, sum, m0, n0, lane);
+  qmm_store_block<NB>(a.y, a.y_dtype, a.M, a.N, sum, m0, n0, lane);
 }
 
 // ---- generic kernel (fp32 / bf16 activations) ------------------------------------------
@@ -742,10 +776,12 @@ __global__ void __launch_bounds__(256) qmm_generic_kernel(QmmArgs a) {
 
 namespace gsq {
 
-// Tiles of 192 rows where they cover M with fewer 16-row blocks than tiles of 256 (equal: 256, which
-// decode the weights less often).
+// Tiles of 192 or 256 rows: a column of a tile costs about 4 + its 16-row blocks (the decode and the
+// per-stage work count as four: IQ2_S 17408 x 5120 8.1 us against 10.2), so 192 where that covers M
+// for less (182 rows: 98 -> 76 us with everything else of this plan; 800 rows: 242 us with 192, 228
+// with 256).
 static int qmm_tall_blocks(long long M) {
-  return (M + 191) / 192 * 12 < (M + 255) / 256 * 16 ? 12 : 16;
+  return (M + 191) / 192 * (4 + 12) < (M + 255) / 256 * (4 + 16) ? 12 : 16;
 }
 
 // ---- host side --------------------------------------------------------------------------
@@ -759,31 +795,33 @@ static bool qmm_grid_type(int qt) {
 // Launch plans of the tiled kernel: ring height MF and tile height MC (16-row blocks) and waves.
 // MF 16 holds tiles of 16 or 12 blocks (192 rows), so that 129-192 rows (and the like of larger
 // batches) do not multiply padding.
-template <int T, int MF, int MC, int WV>
-static hipError_t launch_mfma_t(QmmMfmaArgs a, bool a4, hipStream_t s) {
+template <int T, int MF, int MC, bool A4, int WV>
+static hipError_t launch_mfma_k(const QmmMfmaArgs& a, hipStream_t s) {
   using Plan = QmmPlan<T, MF, WV>;
   static_assert(Plan::kValid);
+  auto k = qmm_mfma_kernel<T, MF, MC, A4, WV>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kQLds - Plan::kTbl);
+    if (e != hipSuccess) return e;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(k, dim3(a.G), dim3(64 * WV), Plan::kLds - Plan::kTbl, s, a);
+  return hipGetLastError();
+}
+
+template <int T, int MF, int MC, int WV>
+static hipError_t launch_mfma_t(const QmmMfmaArgs& a, bool a4, hipStream_t s) {
   constexpr int NB = QmmGeo<T, WV>::kNB;
-  constexpr size_t lds = Plan::kLds - Plan::kTbl;  // dynamic part
-  auto go = [&](auto k) -> hipError_t {
-    static bool attr_set = false;
-    if (!attr_set) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kQLds - Plan::kTbl);
-      if (e != hipSuccess) return e;
-      attr_set = true;
-    }
-    hipLaunchKernelGGL(k, dim3(a.G), dim3(64 * WV), lds, s, a);
-    return hipGetLastError();
-  };
   hipError_t e;
   if constexpr (BlockBytes<T>::v % 4 == 0) {
-    e = a4 ? go(qmm_mfma_kernel<T, MF, MC, true, WV>) : go(qmm_mfma_kernel<T, MF, MC, false, WV>);
+    e = a4 ? launch_mfma_k<T, MF, MC, true, WV>(a, s) : launch_mfma_k<T, MF, MC, false, WV>(a, s);
   } else {
-    e = go(qmm_mfma_kernel<T, MF, MC, false, WV>);
+    e = launch_mfma_k<T, MF, MC, false, WV>(a, s);
   }
-  // split tiles: unless every workgroup's range starts at a tile's first column
-  if (e == hipSuccess && a.G > 1 && ((long long)a.units % a.G != 0 || (a.units / a.G) % a.nblk != 0)) {
-    hipLaunchKernelGGL((qmm_reduce_kernel<MC, NB, WV>), dim3(a.G - 1, MC), dim3(64 * WV), 0, s, a);
+  // unless every range starts at a tile's first column
+  if (e == hipSuccess && a.GS > 1 && (a.units % a.GS != 0 || (a.units / a.GS) % a.nblk != 0)) {
+    hipLaunchKernelGGL((qmm_reduce_kernel<T, MC, NB, WV>), dim3(a.GS - 1, MC), dim3(64 * WV), 0, s, a);
     e = hipGetLastError();
   }
   return e;
@@ -809,15 +847,20 @@ static hipError_t launch_mfma(QmmMfmaArgs& a, int num_cus, const QmmWorkspace& w
     // weight tile fastest: the workgroups of one XCD (consecutive units) share an activation
     // tile in its L2 (3-6% faster at M = 2048 than activation tile fastest)
     a.nfast = g_qmm_tuning.order == 2 ? 0 : 1;
-    const long long units = (long long)a.mt * a.nt * a.nblk;
-    if (units >= (1ll << 31)) return hipErrorInvalidValue;
-    a.units = (int)units;
-    const int gmax = (a.units + min_cols - 1) / min_cols;
-    a.G = num_cus < gmax ? num_cus : gmax;
-    if (a.G > ws.max_groups) a.G = ws.max_groups;
+    const long long tiles = (long long)a.mt * a.nt;
+    if (tiles * a.nblk >= (1ll << 31)) return hipErrorInvalidValue;
+    const int cap = num_cus < ws.max_groups ? num_cus : ws.max_groups;
+    const int gmax = (int)((tiles * a.nblk + min_cols - 1) / min_cols);
+    a.G = cap < gmax ? cap : gmax;
+    // whole tiles first: 2048 rows of 17408 x 5120 (544 tiles on 256 CUs) go through 287 partial
+    // tiles instead of 480
+    a.rounds = (int)(tiles / a.G);
+    a.units = (int)(tiles - (long long)a.rounds * a.G) * a.nblk;
+    const int smax = (a.units + min_cols - 1) / min_cols;
+    a.GS = a.G < smax ? a.G : smax;
     // a workspace too small for this tile height's partials at this grid: lower tiles
     a.slot_floats = mc * 16 * kQBN;
-    if (2ll * a.G * a.slot_floats * 4 <= ws.part_bytes) break;
+    if (2ll * a.GS * a.slot_floats * 4 <= ws.part_bytes) break;
     if (mc == 4) return hipErrorInvalidValue;
     mc = mc > 8 ? 8 : 4;
   }
