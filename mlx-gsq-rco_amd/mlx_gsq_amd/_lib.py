@@ -96,8 +96,28 @@ def ensure_tables(qtype: str, device: torch.device) -> None:
     _uploaded[key] = _tables.version()
 
 
+# the current stream's handle by device index, without building a Stream object (a quarter of a
+# small product's host time)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
+
+
+def launch(name: str, device: torch.device, args: tuple, what: str) -> None:
+    """``name(*args, stream)`` on ``device`` (a tensor's) and its current stream. The device is
+    switched only when it is not the current one: entering and leaving the context costs as much
+    as the launch itself."""
+    fn = getattr(_lib or lib(), name)
+    if torch.cuda.current_device() == device.index:
+        rc = fn(*args, _raw_stream(device.index))
+    else:
+        with torch.cuda.device(device):
+            rc = fn(*args, _raw_stream(device.index))
+    if rc != GSQ_OK:
+        check(rc, what)
 
 
 def prepare(device=None, stream=None) -> None:

@@ -31,13 +31,12 @@ def iq2_s_embedding(ids, packed, *, vocab_size: int, dimensions: int, dtype=None
         raise TypeError(f"ids must be int32 or int64, got {ids.dtype}")
     if ids.device.type != "cuda" or packed.device != ids.device:
         raise ValueError("ids and packed must be on the same GPU device")
-    flat = ids.reshape(-1).contiguous()
-    out = torch.empty((flat.numel(), dimensions), dtype=dtype, device=ids.device)
-    if flat.numel():
+    ids = ids.contiguous()
+    out = torch.empty(ids.shape + (dimensions,), dtype=dtype, device=ids.device)
+    if ids.numel():
         _lib.ensure_tables("IQ2_S", ids.device)
-        with torch.cuda.device(ids.device):
-            _lib.check(_lib.lib().gsq_embedding(TYPE_IDS["IQ2_S"], packed.contiguous().data_ptr(), flat.data_ptr(),
-                                                _lib.ID_CODES[flat.dtype], flat.numel(), vocab_size, dimensions,
-                                                out.data_ptr(), _lib.DTYPE_CODES[dtype], _lib.stream_handle(ids.device)),
-                       "iq2_s_embedding")
-    return out.reshape(*ids.shape, dimensions)
+        packed = packed.contiguous()
+        _lib.launch("gsq_embedding", ids.device, (TYPE_IDS["IQ2_S"], packed.data_ptr(), ids.data_ptr(),
+                                                  _lib.ID_CODES[ids.dtype], ids.numel(), vocab_size, dimensions,
+                                                  out.data_ptr(), _lib.DTYPE_CODES[dtype]), "iq2_s_embedding")
+    return out

@@ -41,17 +41,13 @@ def quantized_matmul(x, packed, *, qtype: str, out_features: int, in_features: i
         raise TypeError(f"unsupported activation dtype {x.dtype}")
     if x.device.type != "cuda" or packed.device != x.device:
         raise ValueError("x and packed must be on the same GPU device")
-    original = x.shape[:-1]
     rows = x.numel() // in_features
-    flat = x.reshape(rows, in_features).contiguous()
-    packed = packed.contiguous()
     odt = out_dtype or x.dtype
-    y = torch.empty((rows, out_features), dtype=odt, device=x.device)
+    y = torch.empty(x.shape[:-1] + (out_features,), dtype=odt, device=x.device)
     if rows:
         _lib.ensure_tables(qtype, x.device)
-        with torch.cuda.device(x.device):
-            _lib.check(_lib.lib().gsq_qmm(TYPE_IDS[qtype], packed.data_ptr(), flat.data_ptr(),
-                                          _lib.DTYPE_CODES[flat.dtype], y.data_ptr(), _lib.DTYPE_CODES[odt],
-                                          rows, out_features, in_features, _lib.stream_handle(x.device)),
-                       "quantized_matmul")
-    return y.reshape(*original, out_features)
+        x, packed = x.contiguous(), packed.contiguous()
+        _lib.launch("gsq_qmm", x.device, (TYPE_IDS[qtype], packed.data_ptr(), x.data_ptr(), _lib.DTYPE_CODES[x.dtype],
+                                          y.data_ptr(), _lib.DTYPE_CODES[odt], rows, out_features, in_features),
+                    "quantized_matmul")
+    return y

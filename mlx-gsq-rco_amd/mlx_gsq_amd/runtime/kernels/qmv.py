@@ -76,27 +76,22 @@ def quantized_matvec(x, packed, *, qtype: str, out_features: int, in_features: i
     dtype ``out_dtype`` (default: ``x.dtype``, as the reference).
     """
     _validate(x, packed, qtype, out_features, in_features)
-    original = x.shape[:-1]
     rows = x.numel() // in_features
-    flat = x.reshape(rows, in_features)
     if routes_to_qmm(rows, x.dtype, out_features, in_features):
-        return quantized_matmul(flat, packed, qtype=qtype, out_features=out_features,
-                                in_features=in_features, out_dtype=out_dtype).reshape(*original, out_features)
+        return quantized_matmul(x, packed, qtype=qtype, out_features=out_features, in_features=in_features,
+                                out_dtype=out_dtype)
     if qtype not in QTYPES:
         raise KeyError(qtype)
     _check_tensors(x, packed)
     odt = out_dtype or x.dtype
-    flat = flat.contiguous()
-    packed = packed.contiguous()
-    y = torch.empty((rows, out_features), dtype=odt, device=x.device)
+    y = torch.empty(x.shape[:-1] + (out_features,), dtype=odt, device=x.device)
     if rows:
         _lib.ensure_tables(qtype, x.device)
-        with torch.cuda.device(x.device):
-            _lib.check(_lib.lib().gsq_qmv(TYPE_IDS[qtype], packed.data_ptr(), flat.data_ptr(),
-                                          _lib.DTYPE_CODES[flat.dtype], y.data_ptr(), _lib.DTYPE_CODES[odt],
-                                          rows, out_features, in_features, _lib.stream_handle(x.device)),
-                       "quantized_matvec")
-    return y.reshape(*original, out_features)
+        x, packed = x.contiguous(), packed.contiguous()
+        _lib.launch("gsq_qmv", x.device, (TYPE_IDS[qtype], packed.data_ptr(), x.data_ptr(), _lib.DTYPE_CODES[x.dtype],
+                                          y.data_ptr(), _lib.DTYPE_CODES[odt], rows, out_features, in_features),
+                    "quantized_matvec")
+    return y
 
 
 def quantized_matvec_group2(x, packed0, packed1, *, qtypes, out_features, in_features: int, out_dtype=None):
