@@ -240,12 +240,21 @@ __device__ __forceinline__ int qmm_row(int j, int r) {
   return 4 * NB * (r >> 2) + 4 * j + (r & 3);
 }
 
-// workgroup whose range holds column u: ranges are [floor(w*units/G), floor((w+1)*units/G))
-__device__ __forceinline__ int qmm_owner(int u, int units, int G) {
-  return (int)(((long long)(u + 1) * G + units - 1) / units) - 1;
-}
+// Ranges are [floor(w * units / G), floor((w + 1) * units / G)), in 32-bit arithmetic (w * (units % G)
+// stays below G^2 < 2^31): the 64-bit divisions of the plain form are a hundred instructions each,
+// in front of a launch's first load and of its last store.
 __device__ __forceinline__ int qmm_first_col(int w, int units, int G) {
-  return (int)((long long)w * units / G);
+  const unsigned q = (unsigned)units / (unsigned)G, r = (unsigned)units - q * (unsigned)G;
+  return (int)((unsigned)w * q + (unsigned)w * r / (unsigned)G);
+}
+// workgroup whose range holds column u: a float estimate (within one: G is at most a few thousand),
+// then the exact bounds
+__device__ __forceinline__ int qmm_owner(int u, int units, int G) {
+  int w = (int)(((float)u + 0.5f) * ((float)G / (float)units));
+  w = w < G ? w : G - 1;
+  while (qmm_first_col(w, units, G) > u) --w;
+  while (qmm_first_col(w + 1, units, G) <= u) ++w;
+  return w;
 }
 
 // A loop over 0 .. N - 1 unrolled at compile time (each index a constant): code over the
@@ -629,14 +638,16 @@ __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) 
 }
 
 // Sums the partials of the split tiles in workgroup order (deterministic) and writes y: one
-// workgroup per (boundary between two workgroups' ranges, 16-row activation block), working only at
-// the first boundary inside each split tile. Its own launch, so that every CU reads partials at
+// workgroup per (boundary between two workgroups' ranges, 16-row activation block, half of the
+// tile's waves), working only at the first boundary inside each split tile, with up to eight
+// partials' loads in flight. Its own launch, so that every CU reads partials at
 // once: summed inside the main kernel by a tile's last workgroup to arrive, one CU read all of a
 // tile's partials (2 to 13 of 128-256 KB) with the others idle, 25-38 us at the end of a launch.
 template <int T, int MC, int NB, int WV>  // T: one kernel symbol per translation unit
-__global__ void __launch_bounds__(64 * WV) qmm_reduce_kernel(QmmMfmaArgs a) {
-  constexpr int TH = 64 * WV, UN = 4;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = blockIdx.y;
+__global__ void __launch_bounds__(256) qmm_reduce_kernel(QmmMfmaArgs a) {
+  constexpr int TH = 64 * WV, UN = 8;
+  // four of the main kernel's waves per workgroup
+  const int tid = blockIdx.z * 256 + threadIdx.x, lane = tid & 63, wave = tid >> 6, i = blockIdx.y;
   const int w = (int)blockIdx.x + 1, ub = qmm_first_col(w, a.units, a.GS), st = ub / a.nblk;  // st: split tile
   if (ub == st * a.nblk || qmm_first_col(w - 1, a.units, a.GS) > st * a.nblk) return;
   const int tile = a.rounds * a.G + st;
@@ -655,11 +666,12 @@ __global__ void __launch_bounds__(64 * WV) qmm_reduce_kernel(QmmMfmaArgs a) {
   for (int v = wf; v <= wl; v += UN) {
     float4_t ld[UN][NB];
 #pragma unroll
-    for (int u = 0; u < UN; ++u) {  // clamped to the last piece: its repeats are not added
-      const float* p = slot(v + u <= wl ? v + u : wl);
+    for (int u = 0; u < UN; ++u)
+      if (v + u <= wl) {
+        const float* p = slot(v + u);
 #pragma unroll
-      for (int j = 0; j < NB; ++j) ld[u][j] = *reinterpret_cast<const float4_t*>(p + (size_t)j * TH * 4);
-    }
+        for (int j = 0; j < NB; ++j) ld[u][j] = *reinterpret_cast<const float4_t*>(p + (size_t)j * TH * 4);
+      }
 #pragma unroll
     for (int u = 0; u < UN; ++u)
       if (v + u <= wl) {
@@ -821,7 +833,7 @@ static hipError_t launch_mfma_t(const QmmMfmaArgs& a, bool a4, hipStream_t s) {
   }
   // unless every range starts at a tile's first column
   if (e == hipSuccess && a.GS > 1 && (a.units % a.GS != 0 || (a.units / a.GS) % a.nblk != 0)) {
-    hipLaunchKernelGGL((qmm_reduce_kernel<T, MC, NB, WV>), dim3(a.GS - 1, MC), dim3(64 * WV), 0, s, a);
+    hipLaunchKernelGGL((qmm_reduce_kernel<T, MC, NB, WV>), dim3(a.GS - 1, MC, WV / 4), dim3(256), 0, s, a);
     e = hipGetLastError();
   }
   return e;
