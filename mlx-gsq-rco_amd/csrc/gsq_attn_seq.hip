@@ -9,10 +9,11 @@
 // Before, the torch formulation took tens of launches, float32 copies of the caches, two float32
 // GEMMs over all max_len positions and several passes over a (heads, tokens, max_len) float32
 // score matrix: ~1790 us of a layer over 1024 tokens with a 4096-position cache (24 heads of 256);
-// these two kernels 26 + 72 us.
+// these two kernels 22 + 51 us.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "gsq_common.h"
 
@@ -22,6 +23,9 @@ namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -34,7 +38,10 @@ struct A16;
 template <>
 struct A16<false> {
   static constexpr int kTerms = 2;
-  static constexpr float kScale = 16384.f;
+  static constexpr float kScale = 14.f;  // log2
+  // two values rounded to nearest, and as a pair of floats again
+  __device__ static uint32_t pack(f32x2 v) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2)); }
+  __device__ static f32x2 unpack(uint32_t w) { return __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2); }
   __device__ static float ld(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
   __device__ static uint16_t mk(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
   __device__ static f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
@@ -44,7 +51,9 @@ struct A16<false> {
 template <>
 struct A16<true> {
   static constexpr int kTerms = 3;
-  static constexpr float kScale = 1.f;
+  static constexpr float kScale = 0.f;
+  __device__ static uint32_t pack(f32x2 v) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2)); }
+  __device__ static f32x2 unpack(uint32_t w) { return (f32x2){ld((uint16_t)w), ld((uint16_t)(w >> 16))}; }
   __device__ static float ld(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
   __device__ static uint16_t mk(float v) { return (uint16_t)f32_to_bf16_bits(v); }
   __device__ static f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
@@ -63,6 +72,9 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// v_exp_f32: 2^x to one ulp (results below the normal range are 0)
+__device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
+
 // Transposing LDS read: 16 lanes read 4 rows of 16 values (lane j: values 4 (j % 4) .. + 3 of row
 // j / 4, 8 bytes); lane j gets column j of the four rows.
 __device__ __forceinline__ s16x4 tr_read(const uint8_t* p) {
@@ -71,69 +83,100 @@ __device__ __forceinline__ s16x4 tr_read(const uint8_t* p) {
 
 }  // namespace
 
-// One workgroup per token: the rotary factors of its position once (angles in double, as the
-// single-token kernels form them), then a wave per head over the query and key heads: RMS norm and
-// rounding, rotate-half on the first rd dims and rounding; k and v go into the caches, q to scratch
-// as (B, H, S, hd). Bound by memory (q, k, v read once and written once).
-template <bool BF>
+// One workgroup per token: a wave per head over the query and key heads, kPrepHeads at a time, all
+// their loads issued before the rotary factors of the position are formed (angles in double, as
+// the single-token kernels form them) and before any is used: RMS norm and rounding, rotate-half
+// on the first rd dims and rounding; k and v go into the caches, q to scratch as (B, H, S, hd).
+// Bound by memory latency (q, k, v read once and written once): 1024 tokens of 28 heads of 256 took
+// 28 us with each head's loads waited for in turn, 22 so.
+constexpr int kPrepHeads = 8;
+
+template <bool BF, int HD>
 __global__ void __launch_bounds__(256) attn_prep_seq_kernel(AttnSeqArgs a) {
   using E = A16<BF>;
-  __shared__ float row[4][256], cs[128], sn[128];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int t = blockIdx.x, bb = blockIdx.y, hd = a.hd, rd = a.rd, hr = rd / 2;
+  constexpr int V = HD / 64;  // consecutive values per lane
+  typedef uint16_t vec_t __attribute__((ext_vector_type(V)));
+  __shared__ float row[4][HD], cs[HD / 2], sn[HD / 2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, d0 = V * lane;
+  const int t = blockIdx.x, bb = blockIdx.y, rd = a.rd, hr = rd / 2, nh = a.H + a.Hkv;
   if (seq_pos_invalid(a)) return;
   const int64_t p = a.pos[0] + t, r = (int64_t)bb * a.S + t;
-  if (tid < hr) {
-    const double ang = (double)p * a.inv_freq[tid];
-    cs[tid] = (float)cos(ang);
-    sn[tid] = (float)sin(ang);
+  const uint16_t* qg = static_cast<const uint16_t*>(a.qg) + r * a.qg_stride + d0;
+  const uint16_t* kn = static_cast<const uint16_t*>(a.k) + r * a.k_stride + d0;
+  const uint16_t* vn = static_cast<const uint16_t*>(a.v) + r * a.v_stride + d0;
+  float wq[V], wk[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    wq[j] = E::ld(static_cast<const uint16_t*>(a.q_norm_w)[d0 + j]);
+    wk[j] = E::ld(static_cast<const uint16_t*>(a.k_norm_w)[d0 + j]);
   }
-  __syncthreads();
-  const uint16_t* qg = static_cast<const uint16_t*>(a.qg) + r * a.qg_stride;
-  const uint16_t* kn = static_cast<const uint16_t*>(a.k) + r * a.k_stride;
-  const uint16_t* vn = static_cast<const uint16_t*>(a.v) + r * a.v_stride;
-  for (int h = wave; h < a.H + a.Hkv; h += 4) {
-    const bool isq = h < a.H;
-    const int kh = h - a.H;
-    const uint16_t* src = isq ? qg + (int64_t)h * 2 * hd : kn + (int64_t)kh * hd;
-    const uint16_t* w = static_cast<const uint16_t*>(isq ? a.q_norm_w : a.k_norm_w);
-    const int64_t cache = (((int64_t)bb * a.Hkv + kh) * a.L + p) * hd;
-    uint16_t* dst = isq ? static_cast<uint16_t*>(a.q) + (((int64_t)bb * a.H + h) * a.S + t) * hd
-                        : static_cast<uint16_t*>(a.kc) + cache;
-    float x[4], wv[4], ss = 0.f;
+  for (int h0 = wave; h0 < nh; h0 += 4 * kPrepHeads) {
+    uint16_t x[kPrepHeads][V];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = lane + 64 * j;
-      x[j] = d < hd ? E::ld(src[d]) : 0.f;
-      wv[j] = d < hd ? E::ld(w[d]) : 0.f;
-      ss += x[j] * x[j];
+    for (int u = 0; u < kPrepHeads; ++u) {
+      const int h = min(h0 + 4 * u, nh - 1);
+      const uint16_t* src = h < a.H ? qg + (int64_t)h * 2 * HD : kn + (int64_t)(h - a.H) * HD;
+#pragma unroll
+      for (int j = 0; j < V; ++j) x[u][j] = src[j];
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-    const float rn = 1.f / sqrtf(ss / (float)hd + a.eps);
-    // the wave's own row area: its LDS operations complete in order
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (lane + 64 * j < hd) row[wave][lane + 64 * j] = x[j] = E::ld(E::mk(x[j] * rn * wv[j]));
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = lane + 64 * j;
-      if (d >= hd) continue;
-      float v = x[j];
-      if (d < rd) {
-        const int i = d < hr ? d : d - hr;
-        const float other = d < hr ? -row[wave][d + hr] : row[wave][i];
-        v = v * cs[i] + other * sn[i];
+    if (h0 == wave) {
+      if (tid < hr) {
+        const double ang = (double)p * a.inv_freq[tid];
+        cs[tid] = (float)cos(ang);
+        sn[tid] = (float)sin(ang);
       }
-      dst[d] = E::mk(v);
-      if (!isq) static_cast<uint16_t*>(a.vc)[cache + d] = vn[(int64_t)kh * hd + d];
+      __syncthreads();
     }
-    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < kPrepHeads; ++u) {
+      const int h = h0 + 4 * u, kh = h - a.H;
+      if (h >= nh) break;
+      const bool isq = h < a.H;
+      const int64_t cache = (((int64_t)bb * a.Hkv + kh) * a.L + p) * HD + d0;
+      uint16_t* dst = isq ? static_cast<uint16_t*>(a.q) + (((int64_t)bb * a.H + h) * a.S + t) * HD + d0
+                          : static_cast<uint16_t*>(a.kc) + cache;
+      float f[V], ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        f[j] = E::ld(x[u][j]);
+        ss += f[j] * f[j];
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      const float rn = 1.f / sqrtf(ss / (float)HD + a.eps);
+      // the wave's own row area: its LDS operations complete in order
+#pragma unroll
+      for (int j = 0; j < V; ++j) row[wave][d0 + j] = f[j] = E::ld(E::mk(f[j] * rn * (isq ? wq[j] : wk[j])));
+      __builtin_amdgcn_wave_barrier();
+      vec_t o;
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        const int d = d0 + j;
+        float v = f[j];
+        if (d < rd) {
+          const int i = d < hr ? d : d - hr;
+          const float other = d < hr ? -row[wave][d + hr] : row[wave][i];
+          v = v * cs[i] + other * sn[i];
+        }
+        o[j] = E::mk(v);
+      }
+      *reinterpret_cast<vec_t*>(dst) = o;
+      if (!isq) {
+        vec_t vv;
+#pragma unroll
+        for (int j = 0; j < V; ++j) vv[j] = vn[(int64_t)kh * HD + j];
+        *reinterpret_cast<vec_t*>(static_cast<uint16_t*>(a.vc) + cache) = vv;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 }
 
-// 64 query tokens of one head per workgroup, 16 per wave, over tiles of 64 cached positions.
+// 64 query tokens of one head per workgroup, 16 per wave, over tiles of 64 cached positions: two
+// groups of four waves take the even and the odd tiles, and their maxima, sums and outputs are
+// merged at the end (a prompt's last query tile is a chain of all its key tiles, and
+// that chain is the kernel's time: 1024 tokens of 24 heads of 256, 72 us with one group and two
+// workgroups per CU, 51 with two and the powers of two below).
 //
 //  * Both products are formed transposed: S^T = K Q^T puts a query on each lane column (lane % 16)
 //    and keys 4 (lane / 16) + e of every 16-key block on its registers, which is what the B operand
@@ -143,29 +186,30 @@ __global__ void __launch_bounds__(256) attn_prep_seq_kernel(AttnSeqArgs a) {
 //  * P stays at fp32 accuracy: 2 fp16 or 3 bf16 terms (A16), each its own MFMA; K, V and Q are the
 //    16-bit values the caches hold, so the products with them are exact.
 //  * K and V tiles come by DMA into one LDS buffer each, V's while the scores are formed and the
-//    next K's while P V is: 64 KB at hd = 256, two workgroups per CU. 16-byte octets are
+//    next K's while P V is: 64 KB a group at hd = 256. 16-byte octets are
 //    XOR-swizzled by key so that the reads are free of bank conflicts; V^T operands are
 //    transposing reads (four keys x 16 dims per 16 lanes).
 //
 // Bound by LDS reads (every wave reads the whole K and V tile: ~2000 cycles a tile of 64 x 64
 // against ~1500 of MFMA); late tiles of the triangle are started first.
 template <bool BF, int HD>
-__global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
+__global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
   using E = A16<BF>;
   constexpr int NO = HD / 8, KS = HD / 32, NI = NO / 4, DB = HD / 16, RB = HD * 2;  // RB: bytes of a row
   constexpr int SH = HD == 64 ? 1 : 0;  // 128-byte rows: two rows to the 64 banks
   // dynamic LDS: reads of a static array would wait for every DMA in flight, the other buffer's too
   extern __shared__ __attribute__((aligned(16))) uint8_t attn_lds[];
-  uint8_t* const kt = attn_lds;
-  uint8_t* const vt = attn_lds + 64 * RB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave8 & 3, grp = wave8 >> 2;
+  uint8_t* const kt = attn_lds + grp * 128 * RB;
+  uint8_t* const vt = kt + 64 * RB;
   const int g = lane >> 4, c = lane & 15;
   const int ntile = (a.S + 63) / 64, h = blockIdx.x % a.H, tile = ntile - 1 - blockIdx.x / a.H, bb = blockIdx.y;
   const int t0 = tile * 64, tw = t0 + 16 * wave, t = min(tw + c, a.S - 1);  // rows past S repeat the last
   const bool on = tw + c < a.S;
   uint16_t* const out = static_cast<uint16_t*>(a.out) + ((int64_t)bb * a.S + t) * a.out_stride + (int64_t)h * HD;
   if (seq_pos_invalid(a)) {
-    if (on)
+    if (on && grp == 0)
       for (int i = 0; i < DB; ++i)
         for (int e = 0; e < 4; ++e) out[16 * i + 4 * g + e] = E::mk(__builtin_nanf(""));
     return;
@@ -184,8 +228,8 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
                                        (lds_ptr_t)(dst + (wave * NI + i) * 1024), 16, 0, 0);
     }
   };
-  issue(Kg, kt, 0, ksw);
-  issue(Vg, vt, 0, vsw);
+  issue(Kg, kt, 64 * grp, ksw);
+  issue(Vg, vt, 64 * grp, vsw);
   u32x4 qf[KS];
   {
     const uint16_t* q = static_cast<const uint16_t*>(a.q) + (((int64_t)bb * a.H + h) * a.S + t) * HD + 8 * g;
@@ -196,7 +240,9 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
 #pragma unroll
   for (int i = 0; i < DB; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;  // l: this lane's share of the row sum
-  const float scale = 1.f / sqrtf((float)HD);
+  // probabilities as powers of two of one fused multiply-add: the products are not rounded before the
+  // maximum is taken off, and the rounding of (maximum x c) is common to a row
+  const float c_ = 1.44269504088896340736f / sqrtf((float)HD);
   const int qpos = pos + t, wmin = pos + min(tw, a.S - 1), wmax = pos + min(tw + 15, a.S - 1);
   const int nk = (pos + min(t0 + 63, a.S - 1)) / 64 + 1;
   // lane bases of the K and V reads (their swizzles depend on the lane only)
@@ -205,9 +251,9 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
   const uint8_t* const vb = vt + vkey * RB + (((c & 3) >> 1) << 4) + ((c & 1) << 3);
   // the query fragments (loaded after the tiles' DMA) are in registers before the loop counts loads
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  for (int kt0 = 0; kt0 < nk; ++kt0) {
-    const int k0 = kt0 * 64;
-    const bool live = k0 <= wmax, more = kt0 + 1 < nk;  // a tile past the wave's last position: barriers only
+  for (int kt0 = 0; kt0 < nk; kt0 += 2) {
+    const int k0 = (kt0 + grp) * 64;
+    const bool live = k0 <= wmax, more = kt0 + 2 < nk;  // a tile past the wave's last position: barriers only
     wait_vm<NI>();  // K has landed (V's DMA may be in flight)
     asm volatile("s_barrier" ::: "memory");
     f32x4 s[4];
@@ -221,7 +267,7 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with K
-    if (more) issue(Kg, kt, k0 + 64, ksw);
+    if (more) issue(Kg, kt, k0 + 128, ksw);
     u32x4 pf[E::kTerms][2];
     if (live) {
       float mx = -INFINITY;
@@ -229,21 +275,20 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
       for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          s[b][e] *= scale;
           if (k0 + 63 > wmin && k0 + 16 * b + 4 * g + e > qpos) s[b][e] = -INFINITY;
           mx = fmaxf(mx, s[b][e]);
         }
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float mn = fmaxf(m, mx), ms = mn == -INFINITY ? 0.f : mn;
-      const float alpha = expf(m - ms);
+      const float alpha = exp2_raw((m - ms) * c_), off = E::kScale - ms * c_;
       m = mn;
       float sum = 0.f;
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          s[b][e] = expf(s[b][e] - ms) * E::kScale;
+          s[b][e] = exp2_raw(__builtin_fmaf(s[b][e], c_, off));
           sum += s[b][e];
         }
       l = l * alpha + sum;
@@ -257,11 +302,15 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
         for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {  // a pair of k-slots
-            float* v = &(reinterpret_cast<float*>(&s[2 * hf + (j >> 1)])[2 * (j & 1)]);
-            const uint16_t lo = E::mk(v[0]), hi = E::mk(v[1]);
-            pf[n][hf][j] = (uint32_t)lo | ((uint32_t)hi << 16);
-            v[0] -= E::ld(lo);
-            v[1] -= E::ld(hi);
+            f32x4& v = s[2 * hf + (j >> 1)];
+            const f32x2 p2 = j & 1 ? v.zw : v.xy;
+            const uint32_t w = E::pack(p2);
+            pf[n][hf][j] = w;
+            if (n + 1 < E::kTerms) {  // what the term leaves, for the next one
+              const f32x2 left = p2 - E::unpack(w);
+              if (j & 1) v.zw = left;
+              else v.xy = left;
+            }
           }
     }
     if (more) wait_vm<NI>();  // V has landed (the next K's DMA may be in flight)
@@ -283,21 +332,36 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with V
-    if (more) issue(Vg, vt, k0 + 64, vsw);
+    if (more) issue(Vg, vt, k0 + 128, vsw);
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  const float inv = 1.f / l;
+  // merge (every wave is past its last tile read): each group gives its twin lane the other half of
+  // the dims through LDS and finishes its own
+  constexpr int HB = DB / 2;
+  f32x4* const mo = reinterpret_cast<f32x4*>(attn_lds) + wave * HB * 64 + lane;
+  float2* const ml = reinterpret_cast<float2*>(attn_lds + 8 * HB * 1024) + wave * 64 + lane;
+  static_assert(8 * HB * 1024 + 8 * 512 <= 256 * RB);
+#pragma unroll
+  for (int i = 0; i < HB; ++i) mo[grp * 4 * HB * 64 + i * 64] = grp ? acc[i] : acc[HB + i];
+  ml[grp * 256] = make_float2(m, l);
+  __syncthreads();
   if (!on) return;
+  const float2 o1 = ml[(grp ^ 1) * 256];
+  const float mm = fmaxf(m, o1.x), ms = mm == -INFINITY ? 0.f : mm;
+  const float s0 = exp2_raw((m - ms) * c_), s1 = exp2_raw((o1.x - ms) * c_);  // a group without keys: 0 of nothing
+  const float inv = 1.f / (l * s0 + o1.y * s1);
   const uint16_t* gate = static_cast<const uint16_t*>(a.qg) + ((int64_t)bb * a.S + t) * a.qg_stride + (int64_t)h * 2 * HD + HD;
 #pragma unroll
-  for (int i = 0; i < DB; ++i) {
-    const uint2 gw = *reinterpret_cast<const uint2*>(gate + 16 * i + 4 * g);
+  for (int i = 0; i < HB; ++i) {
+    const int d = 16 * (grp * HB + i) + 4 * g;
+    const f32x4 v = (grp ? acc[HB + i] : acc[i]) * s0 + mo[(grp ^ 1) * 4 * HB * 64 + i * 64] * s1;
+    const uint2 gw = *reinterpret_cast<const uint2*>(gate + d);
     const uint16_t gv[4] = {(uint16_t)gw.x, (uint16_t)(gw.x >> 16), (uint16_t)gw.y, (uint16_t)(gw.y >> 16)};
     uint16_t o[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = E::mk(acc[i][e] * inv * (1.f / (1.f + expf(-E::ld(gv[e])))));
-    *reinterpret_cast<uint2*>(out + 16 * i + 4 * g) =
+    for (int e = 0; e < 4; ++e) o[e] = E::mk(v[e] * inv * (1.f / (1.f + expf(-E::ld(gv[e])))));
+    *reinterpret_cast<uint2*>(out + d) =
         make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
   }
 }
@@ -305,13 +369,21 @@ __global__ void __launch_bounds__(256, 2) attn_seq_kernel(AttnSeqArgs a) {
 template <bool BF>
 static hipError_t launch_attn_seq_t(const AttnSeqArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.S + 63) / 64 * a.H), (unsigned)a.B);
-  const size_t lds = (size_t)a.hd * 256;  // a K and a V tile: 64 rows of 2 hd bytes each
-  hipLaunchKernelGGL(attn_prep_seq_kernel<BF>, dim3((unsigned)a.S, (unsigned)a.B), dim3(256), 0, s, a);
-  if (a.hd == 256) hipLaunchKernelGGL((attn_seq_kernel<BF, 256>), grid, dim3(256), lds, s, a);
-  else if (a.hd == 128) hipLaunchKernelGGL((attn_seq_kernel<BF, 128>), grid, dim3(256), lds, s, a);
-  else if (a.hd == 64) hipLaunchKernelGGL((attn_seq_kernel<BF, 64>), grid, dim3(256), lds, s, a);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+  const dim3 pgrid((unsigned)a.S, (unsigned)a.B);
+  auto launch = [&](auto hd) -> hipError_t {
+    constexpr int HD = decltype(hd)::value;
+    constexpr int lds = 2 * 2 * 64 * HD * 2;  // two groups' K and V tiles: 64 rows of 2 hd bytes each
+    static const hipError_t attr = hipFuncSetAttribute((const void*)attn_seq_kernel<BF, HD>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((attn_prep_seq_kernel<BF, HD>), pgrid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((attn_seq_kernel<BF, HD>), grid, dim3(512), lds, s, a);
+    return hipGetLastError();
+  };
+  if (a.hd == 256) return launch(std::integral_constant<int, 256>{});
+  if (a.hd == 128) return launch(std::integral_constant<int, 128>{});
+  if (a.hd == 64) return launch(std::integral_constant<int, 64>{});
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_attn_seq(bool bf16, const AttnSeqArgs& a, hipStream_t s) {
