@@ -895,33 +895,58 @@ static hipError_t launch_mfma(QmmMfmaArgs& a, int num_cus, const QmmWorkspace& w
 template <int T>
 constexpr bool qms_group_layout() { return T != Q6_K && T != Q2_K; }
 
-template <int T, int WV, int NB>
+template <int T, int WV, int NB, int MB>
 static hipError_t launch_qms_a4(const QmsArgs& a, bool a4, hipStream_t s) {
-  static const int env_hx = [] {
-    const char* v = std::getenv("GSQ_QMS_HX");
-    return v ? std::atoi(v) : -1;
-  }();
-  const bool hx = env_hx < 0 ? qms_group_layout<T>() : env_hx > 0;
-  if constexpr (BlockBytes<T>::v % 4 == 0) {
-    if (a4) return hx ? launch_qms_t<T, true, WV, NB, true>(a, s) : launch_qms_t<T, true, WV, NB, false>(a, s);
+  constexpr bool HX = qms_group_layout<T>();
+  if constexpr (MB == 1) {
+    static const int env_hx = [] {
+      const char* v = std::getenv("GSQ_QMS_HX");
+      return v ? std::atoi(v) : -1;
+    }();
+    if (env_hx >= 0 && (env_hx > 0) != HX) {
+      if constexpr (BlockBytes<T>::v % 4 == 0)
+        if (a4) return launch_qms_t<T, true, WV, NB, !HX, MB>(a, s);
+      return launch_qms_t<T, false, WV, NB, !HX, MB>(a, s);
+    }
   }
-  return hx ? launch_qms_t<T, false, WV, NB, true>(a, s) : launch_qms_t<T, false, WV, NB, false>(a, s);
+  if constexpr (BlockBytes<T>::v % 4 == 0)
+    if (a4) return launch_qms_t<T, true, WV, NB, HX, MB>(a, s);
+  return launch_qms_t<T, false, WV, NB, HX, MB>(a, s);
 }
 
-// Plan and launch the small-batch kernel for type T (M <= 16): row groups of WV * 16 * NB
-// rows (8 waves of 16 rows unless the tuning asks otherwise), units divided over at most one
+// Activation blocks of 16 rows the small-batch kernel takes M rows in, or 0: M > 96 (two launches of
+// 64 rows take as long as one 128-row tile of the tiled kernel: 66 against 58 us on 17408 x 5120
+// Q4_K), or a type whose ring of two columns does not fit beside that many (Q6_K past 64 rows and the
+// IQ1 types past 48, whose superblocks or tables are the largest). Wherever it has a plan it is the
+// faster one: 1024-17408 rows or columns, 17-64 rows 1.7-2.6x, 96 rows 1.2-1.6x.
+template <int T>
+static int qms_blocks(int64_t M) {
+  const int mb = M <= 16 ? 1 : M <= 32 ? 2 : M <= 48 ? 3 : M <= 64 ? 4 : M <= 96 ? 6 : 0;
+  const bool ok = mb == 6   ? QmsPlan<T, 8, 1, 6>::kValid
+                  : mb == 4 ? QmsPlan<T, 8, 1, 4>::kValid
+                  : mb == 3 ? QmsPlan<T, 8, 1, 3>::kValid
+                            : mb > 0 && QmsPlan<T, 8, 1, 2>::kValid;
+  return ok ? mb : 0;
+}
+
+// Plan and launch the small-batch kernel for type T (qms_blocks(M) > 0): row groups of WV * 16 * NB
+// weight rows (8 waves of 16 rows unless the tuning asks otherwise), units divided over at most one
 // workgroup per CU, at least min_cols columns each.
 template <int T>
 static hipError_t launch_qms(QmsArgs& a, int num_cus, const QmmWorkspace& ws, hipStream_t s) {
   if (a.tbl_bytes != qmm_tbl_bytes<T>()) return hipErrorInvalidValue;
-  // 16 waves of 16 rows on products of at least 2^26 weights (the 17408-row and 17408-wide 27B
-  // projections: 4-10% faster than 8 waves, whose two waves per SIMD leave the decode's LDS and
-  // MFMA latency exposed; the smaller products, with fewer row groups per CU, are faster with 8)
-  const bool big = (long long)a.N * a.K >= (1ll << 26) && QmsPlan<T, 16, 1>::kValid;
-  const int wv = g_qmm_tuning.small_waves == 4 ? 4
+  const int mb = qms_blocks<T>(a.M);
+  // 16 waves of 16 rows on products of at least 2^26 weights and up to 16 activation rows (the
+  // 17408-row and 17408-wide 27B projections: 4-10% faster than 8 waves, whose two waves per SIMD
+  // leave the decode's LDS and MFMA latency exposed; the smaller products, with fewer row groups per
+  // CU, are faster with 8). With more activation rows the MFMAs cover that latency: 8 waves are
+  // within 4% at 32 rows and even at 64.
+  const bool big = mb == 1 && (long long)a.N * a.K >= (1ll << 26) && QmsPlan<T, 16, 1, 1>::kValid;
+  const int wv = mb > 1 ? 8
+               : g_qmm_tuning.small_waves == 4 ? 4
                : g_qmm_tuning.small_waves == 16 ? 16
                : g_qmm_tuning.small_waves == 8 ? 8 : (big ? 16 : 8);
-  const int nb = g_qmm_tuning.small_nb == 2 ? 2 : (g_qmm_tuning.small_nb == 4 ? 4 : 1);
+  const int nb = mb > 1 ? 1 : g_qmm_tuning.small_nb == 2 ? 2 : (g_qmm_tuning.small_nb == 4 ? 4 : 1);
   const int rg = wv * 16 * nb;
   const long long units = (((long long)a.N + rg - 1) / rg) * a.nblk;
   if (units >= (1ll << 31)) return hipErrorInvalidValue;
@@ -930,19 +955,27 @@ static hipError_t launch_qms(QmsArgs& a, int num_cus, const QmmWorkspace& ws, hi
   const int gmax = (a.units + min_cols - 1) / min_cols;
   a.G = num_cus < gmax ? num_cus : gmax;
   if (a.G > ws.max_groups) a.G = ws.max_groups;
-  // the partials of G workgroups must fit the workspace (slot: NB * 64 * WV float4)
-  while (a.G > 1 && 2ll * a.G * (nb * 64 * wv * 16) > ws.part_bytes) --a.G;
+  // the partials of G workgroups must fit the workspace (slot: MB * NB * 64 * WV float4)
+  while (a.G > 1 && 2ll * a.G * (mb * nb * 64 * wv * 16) > ws.part_bytes) --a.G;
   a.xcd_remap = (a.G % 8 == 0) ? 1 : 0;
   a.part = ws.part;
   a.part_bytes = ws.part_bytes;
   a.cnt = ws.cnt;
   const bool a4 = (reinterpret_cast<uintptr_t>(a.packed) & 3) == 0;
-  if (wv == 16) return launch_qms_a4<T, 16, 1>(a, a4, s);
+  switch (mb) {
+    case 1: break;
+    case 2: return launch_qms_a4<T, 8, 1, 2>(a, a4, s);
+    case 3: return launch_qms_a4<T, 8, 1, 3>(a, a4, s);
+    case 4: return launch_qms_a4<T, 8, 1, 4>(a, a4, s);
+    case 6: return launch_qms_a4<T, 8, 1, 6>(a, a4, s);
+    default: return hipErrorInvalidValue;
+  }
+  if (wv == 16) return launch_qms_a4<T, 16, 1, 1>(a, a4, s);
   if (wv == 8)
-    return nb == 4 ? launch_qms_a4<T, 8, 4>(a, a4, s) : nb == 2 ? launch_qms_a4<T, 8, 2>(a, a4, s)
-                                                                 : launch_qms_a4<T, 8, 1>(a, a4, s);
-  return nb == 4 ? launch_qms_a4<T, 4, 4>(a, a4, s) : nb == 2 ? launch_qms_a4<T, 4, 2>(a, a4, s)
-                                                               : launch_qms_a4<T, 4, 1>(a, a4, s);
+    return nb == 4 ? launch_qms_a4<T, 8, 4, 1>(a, a4, s) : nb == 2 ? launch_qms_a4<T, 8, 2, 1>(a, a4, s)
+                                                                   : launch_qms_a4<T, 8, 1, 1>(a, a4, s);
+  return nb == 4 ? launch_qms_a4<T, 4, 4, 1>(a, a4, s) : nb == 2 ? launch_qms_a4<T, 4, 2, 1>(a, a4, s)
+                                                                 : launch_qms_a4<T, 4, 1, 1>(a, a4, s);
 }
 
 template <int T>
@@ -956,9 +989,9 @@ template <int T>
 static hipError_t launch_qmm_type(const uint8_t* packed, const void* x, int xdt, void* y, int ydt, int64_t M,
                                   int64_t N, int K, const DevTables& tb, int num_cus, const QmmWorkspace& ws,
                                   hipStream_t s) {
-  const int small_max = g_qmm_tuning.small_max_m == 0 ? 16 : g_qmm_tuning.small_max_m;
+  const bool small = M >= 1 && (g_qmm_tuning.small_max_m == 0 || M <= g_qmm_tuning.small_max_m) && qms_blocks<T>(M) > 0;
   const bool x16 = (reinterpret_cast<uintptr_t>(x) & 15) == 0;  // the MFMA kernels read 16-byte pieces
-  if (xdt == QDT_F16 && x16 && ws.part && M >= 1 && M <= small_max && M <= 16 && N < (1ll << 31)) {
+  if (xdt == QDT_F16 && x16 && ws.part && small && N < (1ll << 31)) {
     QmsArgs a{};
     a.packed = packed;
     a.x = static_cast<const _Float16*>(x);

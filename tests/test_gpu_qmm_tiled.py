@@ -1,5 +1,6 @@
-"""Tiled product at the edges of its tiles (64, 128, 192 and 256 rows; 256 weight rows) and of its plan
-(whole tiles first, then tiles split over workgroups and summed by a second launch).
+"""Products at the edges of their tiles and plans: the small-batch kernel (16, 32, 48, 64 and 96 rows;
+128 weight rows) and the tiled one (64, 128, 192 and 256 rows; 256 weight rows; whole tiles first, then
+tiles split over workgroups and summed by a second launch).
 
 Against the oracle's float32 weights in float64, elementwise. A weight is rounded to fp16 at most
 twice (group scale times value, then superblock scale): 2 * 2^-11 of sum |w x|, or 2^-24 |x| where it
@@ -16,8 +17,14 @@ if not torch.cuda.is_available():
 
 SHAPES = [
     (17, 257, 256),     # one column per tile: nothing to split
+    (32, 129, 512),
+    (33, 128, 2560),    # one row group over ten workgroups
+    (48, 1, 256),
+    (49, 127, 768),
     (64, 255, 512),
-    (65, 515, 1280),    # 128-row tiles, weight rows of odd length
+    (65, 515, 1280),    # six blocks (128-row tiles for Q6_K, IQ1_S), weight rows of odd length
+    (96, 40001, 512),   # several columns and parts of two groups per workgroup
+    (97, 130, 1280),    # 128-row tiles
     (128, 256, 768),
     (129, 771, 768),    # 192-row tiles
     (192, 64, 2560),
