@@ -689,7 +689,7 @@ def run_model_decode(device, max_len=1024, prompt=8, steps=32, batches=(8,)):
         ms_b = step_ms(b)
         res["batched"][f"B={b}"] = {"ms_per_step": round(ms_b, 4), "tokens_per_s": round(b * 1e3 / ms_b, 1)}
     # prefill of the reference's published prompt length (eager: tiled QMM projections, the
-    # GatedDeltaNet sequence kernels, attention on torch ops), logits of every position
+    # GatedDeltaNet sequence and prompt attention kernels), logits of every position
     pms = prefill_ms(182)
     res["prefill"] = {"tokens": 182, "ms": round(pms, 2), "tokens_per_s": round(182e3 / pms, 1)}
     del model, store

@@ -116,8 +116,11 @@ int gsq_qmv_pre(int qtype_id, const void* packed, int pre_op, const void* x, con
  * fp32 partials through a workspace the library keeps per (device, stream) and allocates on
  * the first call on that stream (or in gsq_prepare): calls on one stream run in order and
  * share it, calls on different streams may overlap and never share one. A workspace is 2 slots
- * of 256 x 256 floats per CU plus counters (128 MB on a 256-CU device), held until the process
- * ends, for at most 64 streams per device; the call that makes it synchronizes the device once.
+ * of 256 x 256 floats per CU plus counters (128 MB on a 256-CU device) and, where the device has
+ * room for it, 128 MB in which x that is not 16-byte aligned fp16 is laid out as such (more rows
+ * than fit go in several products; without that area, or with rows wider than it, the generic
+ * kernel reads such x directly). It is held until the process ends, for at most 64 streams per
+ * device; the call that makes it synchronizes the device once.
  * A graph captured from stream S uses S's workspace: its replays must not overlap other QMM
  * work on S or replays of other graphs captured from S. */
 int gsq_qmm(int qtype_id, const void* packed, const void* x, int x_dtype, void* y, int y_dtype,
@@ -132,7 +135,8 @@ int gsq_qmm(int qtype_id, const void* packed, const void* x, int x_dtype, void* 
  * (several streams, concurrent graph nodes) race and give wrong results: serialize them. Fixed
  * tables must exist first (gsq_prepare, gsq_set_tables); a call that would need to build one
  * returns GSQ_E_VALUE instead. Results match gsq_qmm within the QMM tolerance (bit for bit
- * where both pick the same tile plan, as for M <= 64). */
+ * where both pick the same tile plan, as for M <= 64 rows of 16-byte aligned fp16 x; other x takes
+ * the generic kernel here). */
 int gsq_qmm_noalloc(int qtype_id, const void* packed, const void* x, int x_dtype, void* y, int y_dtype,
                     int64_t M, int64_t N, int64_t K, void* stream);
 

@@ -6,15 +6,15 @@
 // half, qmm.py:181), activations are staged as fp16 (qmm.py:150-165) and products accumulate
 // in fp32.
 //
-// gfx950 kernel (fp16 activations), one 256-thread workgroup per CU:
-//  * output tile = BM activation rows x 256 weight rows; wave w owns weight rows
-//    [64w, 64w + 64) and all BM rows, so its weights are private to it: the wave decodes them
-//    straight into v_mfma_f32_16x16x32_f16 B operands (lane l: row l%16 of a 16-row block,
+// gfx950 kernel (fp16 activations), one workgroup of 8 waves (4 on 64-row tiles) per CU:
+//  * output tile = BM activation rows x 256 weight rows; wave w owns 32 (64) weight rows of the
+//    tile and all BM rows, so its weights are private to it: the wave decodes them
+//    straight into v_mfma_f32_16x16x32_f16 first operands (lane l: row l%16 of a 16-row block,
 //    weights 8(l/16)..+7 of the 32-weight group) and they never pass through LDS as fp16.
-//  * the wave's 64 superblocks of the current 256-wide K column sit in a private
+//  * the wave's superblocks of the current 256-wide K column sit in a private
 //    two-column LDS ring, filled by global_load_lds DMA one column ahead; each row has a
 //    16-byte aligned slot holding the granules that cover its (2-byte aligned) superblock.
-//  * activations: a ring of `lx` K32 stages of BM x 32 fp16 shared by the four waves, filled
+//  * activations: a ring of `lx` K32 stages of BM x 32 fp16 shared by the waves, filled
 //    by DMA lx-1 stages ahead into a layout whose 16-byte octets are XOR-swizzled per row
 //    (octet o of row m at position o ^ ((m >> 2) & 3)) so that the ds_read_b128 A-operand
 //    reads of a wave are free of bank conflicts.
@@ -29,7 +29,8 @@
 //  * tiles are numbered weight tile fastest and workgroups renumbered so that work done at the
 //    same time (one activation tile, neighbouring weight tiles and K ranges) lands on one XCD and
 //    shares its L2.
-// fp32 / bf16 activations use the generic kernel below.
+// Other activations (fp32, bf16, not 16-byte aligned) are laid out as fp16 in the workspace before
+// this kernel; the generic kernel below serves calls without that area.
 #pragma once
 #include <cstdlib>
 #include <type_traits>
@@ -46,7 +47,7 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 // Final outputs are not read again by the kernel, so fp32 ones are written as streaming
-// (nontemporal) stores; the split-K partials, which the fix-up reads back, keep plain stores.
+// (nontemporal) stores; the split-K partials, which the reduction reads back, keep plain stores.
 __device__ __forceinline__ void qmm_store_y(void* y, int dt, int64_t i, float v) {
   if (dt == QDT_F16) reinterpret_cast<_Float16*>(y)[i] = (_Float16)v;
   else if (dt == QDT_BF16) reinterpret_cast<uint16_t*>(y)[i] = (uint16_t)f32_to_bf16_bits(v);

@@ -5,7 +5,7 @@ same name, keyword arguments (``kt`` is accepted for compatibility; the gfx950 k
 chooses its own K tiling), validation and exceptions. Each wave decodes its own weight rows
 straight from the packed superblocks (DMA'd into LDS) into fp16 MFMA operands in registers,
 once per product, and multiplies them with fp16 activation tiles staged in LDS, accumulating in
-fp32 (libgsq.so; M <= 16 runs a small-batch kernel that decodes every weight once as well).
+fp32 (libgsq.so; up to 96 rows run a small-batch kernel that decodes every weight once as well).
 """
 from __future__ import annotations
 
