@@ -114,8 +114,9 @@ int gsq_qmv_pre(int qtype_id, const void* packed, int pre_op, const void* x, con
 /* Same product with the tiled MFMA kernel (prefill, large M). Replaces quantized_matmul
  * (mlx_gsq/runtime/kernels/qmm.py:559-594). Workgroups that share an output tile exchange
  * fp32 partials through a workspace the library keeps per (device, stream) and allocates on
- * the first call on that stream (or in gsq_prepare): calls on one stream run in order and
- * share it, calls on different streams may overlap and never share one. A workspace is 2 slots
+ * the first call on that stream (or in gsq_prepare): calls on one stream, from any number of host
+ * threads, run in order and share it (the launches of one call are enqueued together), calls on
+ * different streams may overlap and never share one. A workspace is 2 slots
  * of 256 x 256 floats per CU plus counters (128 MB on a 256-CU device) and, where the device has
  * room for it, 128 MB in which x that is not 16-byte aligned fp16 is laid out as such (more rows
  * than fit go in several products; without that area, or with rows wider than it, the generic
@@ -132,7 +133,8 @@ int gsq_qmm(int qtype_id, const void* packed, const void* x, int x_dtype, void* 
  * 32 MiB + 4 KiB that each device holds until the process ends (tile heights are lowered until
  * the partials of one workgroup per CU fit; a device with more than 256 CUs is refused with
  * GSQ_E_VALUE). Every call on a device shares that array, so calls that overlap on one device
- * (several streams, concurrent graph nodes) race and give wrong results: serialize them. Fixed
+ * (several streams, concurrent graph nodes) race and give wrong results: serialize them. Calls on
+ * one stream run in order, whichever threads they come from. Fixed
  * tables must exist first (gsq_prepare, gsq_set_tables); a call that would need to build one
  * returns GSQ_E_VALUE instead. Results match gsq_qmm within the QMM tolerance (bit for bit
  * where both pick the same tile plan, as for M <= 64 rows of 16-byte aligned fp16 x; other x takes

@@ -79,10 +79,19 @@ bool uses_ksigns(int t) { return t == IQ2_XXS || t == IQ2_XS || t == IQ3_XXS; }
 // 1024 workgroups) followed by the split-tile partials of up to 256 workgroups at 64-row
 // activation tiles (2 slots x 64 KiB each); the launch plan lowers the tile height until the
 // partials fit. Every call on a device shares that device's copy: counters are zero when the
-// code object loads and every launch leaves them at zero.
+// code object loads and every call leaves them at zero.
 constexpr size_t kNoAllocCounterBytes = 4096;
 constexpr size_t kNoAllocPartBytes = size_t(32) << 20;
 static __device__ __align__(256) uint8_t scratch[kNoAllocCounterBytes + kNoAllocPartBytes];
+
+// A stream's QMM workspace. A call is up to three launches that pass data through it (activations
+// staged, multiplied, partial tiles summed), so whoever launches on it holds `mu` until the last
+// launch of the call is enqueued: stream order then keeps calls apart, whichever threads they come
+// from.
+struct StreamWorkspace {
+  std::mutex mu;
+  QmmWorkspace ws{};
+};
 
 struct DevState {
   std::map<int, uint16_t*> grids;     // per grid type
@@ -91,9 +100,11 @@ struct DevState {
   uint8_t* ksigns = nullptr;
   int num_cus = 0;
   uint8_t* scratch = nullptr;         // this device's address of `scratch`
-  // QMM workspaces, one per stream: launches on one stream run in order, so they may share
-  // a workspace; launches on different streams may overlap and never share one
-  std::map<hipStream_t, QmmWorkspace> qmm_ws;
+  std::mutex scratch_mu;              // held while the launches of a call that uses it are enqueued
+  // QMM workspaces, one per stream: calls on one stream run in order, so they may share
+  // a workspace; calls on different streams may overlap and never share one. Entries are never
+  // erased and keep their addresses.
+  std::map<hipStream_t, StreamWorkspace> qmm_ws;
 };
 
 // True if `s` is capturing into a HIP graph: nothing may be allocated or copied
@@ -196,15 +207,15 @@ long long qmm_ws_part_bytes(int num_cus) { return 2ll * num_cus * 256 * 256 * (l
 constexpr long long kQmmStageBytes = 128ll << 20;
 
 // The QMM workspace of stream `s` on the current device, allocated on the first QMM call on
-// that stream (or by gsq_prepare); counters start at zero and every launch leaves them at zero.
-int qmm_workspace(hipStream_t s, QmmWorkspace* ws) {
+// that stream (or by gsq_prepare); counters start at zero and every call leaves them at zero.
+int qmm_workspace(hipStream_t s, StreamWorkspace** sw) {
   int dev;
   if (int rc = current_device(&dev)) return rc;
   std::lock_guard<std::mutex> lk(g_mu);
   DevState& st = g_dev[dev];
   auto it = st.qmm_ws.find(s);
   if (it != st.qmm_ws.end()) {
-    *ws = it->second;
+    *sw = &it->second;
     return GSQ_OK;
   }
   if (capturing(s))
@@ -236,13 +247,14 @@ int qmm_workspace(hipStream_t s, QmmWorkspace* ws) {
     xs = nullptr;
     (void)hipGetLastError();
   }
-  *ws = st.qmm_ws[s] = QmmWorkspace{part, cnt, groups, part_bytes, xs, xs ? kQmmStageBytes : 0};
+  *sw = &st.qmm_ws[s];
+  (*sw)->ws = QmmWorkspace{part, cnt, groups, part_bytes, xs, xs ? kQmmStageBytes : 0};
   return GSQ_OK;
 }
 
 // This device's address of `scratch` (host code never passes the symbol itself: on the host it
 // names a shadow variable, not device memory); looked up once per device, with it current.
-int noalloc_scratch(uint8_t** p, int* num_cus) {
+int noalloc_scratch(uint8_t** p, int* num_cus, std::mutex** mu) {
   int dev;
   if (int rc = current_device(&dev)) return rc;
   std::lock_guard<std::mutex> lk(g_mu);
@@ -260,6 +272,7 @@ int noalloc_scratch(uint8_t** p, int* num_cus) {
   }
   *p = st.scratch;
   *num_cus = st.num_cus;
+  *mu = &st.scratch_mu;
   return GSQ_OK;
 }
 
@@ -368,11 +381,12 @@ int gsq_prepare(void* stream) {
     int cus;
     if (int rc = resolve(qt, &tb, &cus, s)) return rc;
   }
-  QmmWorkspace ws;
-  if (int rc = qmm_workspace(s, &ws)) return rc;
+  StreamWorkspace* sw;
+  if (int rc = qmm_workspace(s, &sw)) return rc;
   uint8_t* sp;
   int cus;
-  return noalloc_scratch(&sp, &cus);
+  std::mutex* mu;
+  return noalloc_scratch(&sp, &cus, &mu);
 }
 
 int gsq_tables_ready(int qt) {
@@ -418,10 +432,12 @@ int gsq_qmv(int qt, const void* packed, const void* x, int xdt, void* y, int ydt
     return GSQ_OK;
   }
   // x not 16-byte aligned (the kernels read it in 16-byte pieces): rows are copied into the
-  // stream's QMM workspace first, as many per launch as it holds; stream order keeps the copies
-  // and the launches that read them (and any QMM launch on the stream) apart
-  QmmWorkspace ws;
-  if (int rc = qmm_workspace(s, &ws)) return rc;
+  // stream's QMM workspace first, as many per launch as it holds; the workspace's lock and stream
+  // order keep the copies and the launches that read them (and any QMM call on the stream) apart
+  StreamWorkspace* sw;
+  if (int rc = qmm_workspace(s, &sw)) return rc;
+  std::lock_guard<std::mutex> lk(sw->mu);
+  const QmmWorkspace& ws = sw->ws;
   const int64_t row_bytes = K * xe, chunk = ws.part_bytes / row_bytes;
   if (chunk < 1) return fail(GSQ_E_VALUE, "x row of %lld bytes exceeds the staging workspace", (long long)row_bytes);
   const int64_t ye = ydt == GSQ_F32 ? 4 : 2;
@@ -525,9 +541,10 @@ int gsq_qmm(int qt, const void* packed, const void* x, int xdt, void* y, int ydt
   DevTables tb;
   int cus;
   if (int rc = resolve(qt, &tb, &cus, static_cast<hipStream_t>(stream))) return rc;
-  QmmWorkspace ws;
-  if (int rc = qmm_workspace(static_cast<hipStream_t>(stream), &ws)) return rc;
-  hipError_t e = launch_qmm(qt, static_cast<const uint8_t*>(packed), x, xdt, y, ydt, M, N, (int)K, tb, cus, ws,
+  StreamWorkspace* sw;
+  if (int rc = qmm_workspace(static_cast<hipStream_t>(stream), &sw)) return rc;
+  std::lock_guard<std::mutex> lk(sw->mu);
+  hipError_t e = launch_qmm(qt, static_cast<const uint8_t*>(packed), x, xdt, y, ydt, M, N, (int)K, tb, cus, sw->ws,
                             static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(GSQ_E_HIP, "qmm launch: %s", hipGetErrorString(e));
   return GSQ_OK;
@@ -542,7 +559,8 @@ int gsq_qmm_noalloc(int qt, const void* packed, const void* x, int xdt, void* y,
   int cus;
   if (int rc = resolve(qt, &tb, &cus, s, /*may_alloc=*/false)) return rc;
   uint8_t* sp;
-  if (int rc = noalloc_scratch(&sp, &cus)) return rc;
+  std::mutex* mu;
+  if (int rc = noalloc_scratch(&sp, &cus, &mu)) return rc;
   // the partials of one workgroup per CU at the smallest tile plan (64-row tiles: 2 slots of
   // 64 KiB) must fit the scratch
   const long long need = 2ll * cus * 64 * 1024;
@@ -551,6 +569,7 @@ int gsq_qmm_noalloc(int qt, const void* packed, const void* x, int xdt, void* y,
                 "%zu (use gsq_qmm)", cus, need, kNoAllocPartBytes);
   QmmWorkspace ws{reinterpret_cast<float*>(sp + kNoAllocCounterBytes), reinterpret_cast<int*>(sp),
                   (int)(kNoAllocCounterBytes / sizeof(int)), (long long)kNoAllocPartBytes};
+  std::lock_guard<std::mutex> lk(*mu);
   hipError_t e = launch_qmm(qt, static_cast<const uint8_t*>(packed), x, xdt, y, ydt, M, N, (int)K, tb, cus, ws, s);
   if (e != hipSuccess) return fail(GSQ_E_HIP, "qmm launch: %s", hipGetErrorString(e));
   return GSQ_OK;

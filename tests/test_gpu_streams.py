@@ -3,9 +3,12 @@
 Tiled and small-batch QMM launches exchange split-tile partials through a workspace the library
 keeps per (device, stream), so launches on different streams never share one: the same products
 enqueued concurrently on two streams give the single-stream results bit for bit (the split
-tiles are summed in a fixed order). Capturing QMM on a stream that has no workspace yet fails
+tiles are summed in a fixed order). Several host threads may share one stream: the launches of
+one call are enqueued together. Capturing QMM on a stream that has no workspace yet fails
 cleanly (before anything is enqueued) until gsq_prepare gives it one.
 """
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -78,6 +81,57 @@ def test_qmm_two_streams_concurrently():
             assert torch.equal(c[6], r), f"stream 1, {c[0]}, repeat {rep}"
         for c, r in zip(b, ref_b):
             assert torch.equal(c[6], r), f"stream 2, {c[0]}, repeat {rep}"
+
+
+def test_qmm_threads_share_a_stream():
+    """Threads on one stream, each with calls of several launches over the stream's workspace (split
+    tiles; bf16 and fp32 rows staged as fp16; an unaligned matrix-vector row copied) or the
+    allocation-free entry point's scratch: the single-threaded outputs, bit for bit."""
+    from mlx_gsq_amd import _lib
+    lib = _lib.lib()
+    f16, bf16, f32 = torch.float16, torch.bfloat16, torch.float32
+    specs = [(lib.gsq_qmm, "Q4_K", 200, 1536, 5120, f16, 0), (lib.gsq_qmm, "IQ3_S", 130, 1000, 2048, f16, 0),
+             (lib.gsq_qmm, "Q6_K", 300, 520, 2048, bf16, 0), (lib.gsq_qmm, "IQ2_XS", 20, 1024, 4096, f32, 0),
+             (lib.gsq_qmv, "IQ4_XS", 2, 1024, 5120, f16, 1), (lib.gsq_qmm_noalloc, "Q4_K", 140, 1000, 4096, f16, 0),
+             (lib.gsq_qmm_noalloc, "IQ3_S", 33, 2048, 2048, f16, 0)]
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.prepare()
+    reps, calls = 25, []
+    for i, (fn, qtype, m, n, k, dtype, shift) in enumerate(specs):
+        (_, tid, _, _, pd, _, _, _, _, _), = _cases(((qtype, m, n, k),), 60 + i)
+        flat = torch.randn(m * k + shift, generator=torch.Generator().manual_seed(i)).to(dtype).cuda()
+        x = flat[shift:]
+        y = torch.empty(reps + 1, m, n, device="cuda")
+        calls.append((fn, tid, pd, x, y, m, n, k))
+
+    def enqueue(i, rep):
+        fn, tid, pd, x, y, m, n, k = calls[i]
+        rc = fn(tid, pd.data_ptr(), x.data_ptr(), _lib.DTYPE_CODES[x.dtype], y[rep].data_ptr(), 0, m, n, k, stream)
+        assert rc == 0, lib.gsq_last_error()
+    for i in range(len(calls)):
+        enqueue(i, reps)
+    torch.cuda.synchronize()
+    for c in calls:
+        assert torch.isfinite(c[4][reps]).all()
+    start, failed = threading.Barrier(len(calls)), []
+
+    def work(i):
+        try:
+            start.wait()
+            for rep in range(reps):
+                enqueue(i, rep)
+        except BaseException as e:  # reported by the main thread
+            failed.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed, failed
+    for (_, qtype, m, n, k, dtype, _), c in zip(specs, calls):
+        y = c[4]
+        assert all(torch.equal(y[rep], y[reps]) for rep in range(reps)), (qtype, m, n, k, dtype)
 
 
 def test_qmm_capture_needs_prepared_stream():

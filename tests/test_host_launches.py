@@ -1,0 +1,86 @@
+"""The host side of libgsq.so on a stand-in for the HIP runtime (hip_host_stub.cpp): which launches
+and allocations a call makes. Runs in a child process, where libgsq.so binds to the stand-in."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIB = os.path.join(os.path.dirname(HERE), "mlx-gsq-rco_amd", "mlx_gsq_amd", "libgsq.so")
+
+PRELUDE = """
+import ctypes, sys, threading
+stub = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+stub.stub_malloc_bytes.restype = ctypes.c_size_t
+stub.stub_launch_kernel.restype = ctypes.c_void_p
+I, P, F = ctypes.c_int64, ctypes.c_void_p, ctypes.c_float
+for fn in (lib.gsq_qmm, lib.gsq_qmm_noalloc, lib.gsq_qmv):
+    fn.argtypes = [ctypes.c_int, P, P, ctypes.c_int, P, ctypes.c_int, I, I, I, P]
+lib.gsq_prepare.argtypes = [P]
+lib.gsq_last_error.restype = ctypes.c_char_p
+F32, F16, BF16 = 0, 1, 2
+Q4_K, X, PACKED, Y, S = 12, 1 << 20, 1 << 24, 1 << 28, 1 << 32
+
+def knob(name, value, kind=ctypes.c_int):
+    kind.in_dll(stub, name).value = value
+
+def call(fn, xdt=F16, m=200, n=1536, k=5120, x=X, stream=S):
+    rc = fn(Q4_K, PACKED, x, xdt, Y, F32, m, n, k, stream)
+    assert rc == 0, lib.gsq_last_error()
+
+def counted(fn, *a, **kw):
+    n = stub.stub_launches()
+    call(fn, *a, **kw)
+    return stub.stub_launches() - n
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no g++")
+    so = str(tmp_path_factory.mktemp("stub") / "hip_host_stub.so")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-pthread", "-o", so,
+                    os.path.join(HERE, "hip_host_stub.cpp")], check=True)
+    return so
+
+
+def run(stub, body):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body, stub, LIB], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_launches_of_one_call_stay_together(stub):
+    """Calls that pass data through a stream's workspace (or the allocation-free entry point's scratch)
+    in several launches: another thread's call on that stream never lands between them."""
+    run(stub, """
+lib.gsq_prepare(S)
+# split tiles, summed by a second launch; bf16 and unaligned fp16 rows, laid out by a launch before;
+# an unaligned matrix-vector row, copied by one; and the allocation-free entry point
+CALLS = [(lib.gsq_qmm, {}), (lib.gsq_qmm, dict(xdt=BF16)), (lib.gsq_qmm, dict(x=X + 2, m=20)),
+         (lib.gsq_qmv, dict(x=X + 2, m=1)), (lib.gsq_qmm_noalloc, {}), (lib.gsq_qmm_noalloc, dict(n=1000))]
+lens = [counted(fn, **kw) for fn, kw in CALLS]
+assert lens == [2, 3, 2, 2, 2, 2], lens
+stub.stub_clear()
+knob("stub_launch_us", 100)
+def work(i):
+    stub.stub_thread(i)
+    for _ in range(20):
+        call(CALLS[i][0], **CALLS[i][1])
+threads = [threading.Thread(target=work, args=(i,)) for i in range(len(CALLS))]
+[t.start() for t in threads]
+[t.join() for t in threads]
+log = [stub.stub_launch_thread(i) for i in range(stub.stub_launches())]
+assert len(log) == 20 * sum(lens)
+for group in ({0, 1, 2, 3}, {4, 5}):  # the workspace's users; the scratch's
+    seq = [t for t in log if t in group]
+    i = 0
+    while i < len(seq):
+        n = lens[seq[i]]
+        assert seq[i:i + n] == [seq[i]] * n, f"call of thread {seq[i]} interrupted: {seq[i:i + n]}"
+        i += n
+""")
