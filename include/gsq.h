@@ -58,6 +58,10 @@ int gsq_set_tables(int qtype_id, const float* grid, int64_t entries, int64_t coo
  * counterpart in the reference (MLX compiles and caches its kernels lazily, qmv.py:66). */
 int gsq_prepare(void* stream);
 
+/* gsq_prepare, and the staging area that gsq_qmm on `stream` uses for x that is not 16-byte aligned
+ * fp16 (128 MB, see there): before capturing such calls, or to keep its allocation out of the first. */
+int gsq_prepare_staging(void* stream);
+
 /* 1 if the current device holds the tables `qtype_id` needs, else 0. */
 int gsq_tables_ready(int qtype_id);
 
@@ -117,11 +121,12 @@ int gsq_qmv_pre(int qtype_id, const void* packed, int pre_op, const void* x, con
  * the first call on that stream (or in gsq_prepare): calls on one stream, from any number of host
  * threads, run in order and share it (the launches of one call are enqueued together), calls on
  * different streams may overlap and never share one. A workspace is 2 slots
- * of 256 x 256 floats per CU plus counters (128 MB on a 256-CU device) and, where the device has
- * room for it, 128 MB in which x that is not 16-byte aligned fp16 is laid out as such (more rows
- * than fit go in several products; without that area, or with rows wider than it, the generic
- * kernel reads such x directly). It is held until the process ends, for at most 64 streams per
- * device; the call that makes it synchronizes the device once.
+ * of 256 x 256 floats per CU plus counters (128 MB on a 256-CU device), held until the process
+ * ends, for at most 64 streams per device; the call that makes it synchronizes the device once.
+ * x that is not 16-byte aligned fp16 is laid out as such in another 128 MB, which the first call
+ * on the stream with such x allocates, outside capture (or gsq_prepare_staging; more rows than fit
+ * go in several products). While there is no room for that area, under capture on a stream without
+ * it, or with rows wider than it, the slower generic kernel reads such x directly.
  * A graph captured from stream S uses S's workspace: its replays must not overlap other QMM
  * work on S or replays of other graphs captured from S. */
 int gsq_qmm(int qtype_id, const void* packed, const void* x, int x_dtype, void* y, int y_dtype,

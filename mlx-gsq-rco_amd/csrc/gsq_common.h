@@ -183,7 +183,7 @@ struct AttnSeqArgs {
 
 // QMM workspace: fp32 partial tiles of workgroups that share an output tile (2 slots per
 // workgroup, each sized to the launch plan's tile) and one arrival counter per workgroup, kept
-// at zero between launches. `part_bytes` bounds 2 * groups * slot bytes; `max_groups` bounds the
+// at zero between calls. `part_bytes` bounds 2 * groups * slot bytes; `max_groups` bounds the
 // workgroups (counters). One workspace is never used by two launches that may overlap.
 struct QmmWorkspace {
   float* part;
@@ -193,6 +193,9 @@ struct QmmWorkspace {
   void* xs = nullptr;      // fp16 staging of activations the MFMA kernels cannot read, or null
   long long xs_bytes = 0;
 };
+
+// Whether the MFMA kernels read these activations as they are: fp16 (code 1) at 16-byte pieces.
+inline bool qmm_reads_x(const void* x, int xdt) { return xdt == 1 && (reinterpret_cast<uintptr_t>(x) & 15) == 0; }
 
 // Non-linear IQ4_XS values (k_decode.py:77).
 __device__ __constant__ static const int8_t kIQ4Values[16] = {

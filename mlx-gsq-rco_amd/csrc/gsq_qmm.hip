@@ -119,9 +119,8 @@ static hipError_t launch_qmm_type(int qt, const uint8_t* packed, const void* x, 
 // without a staging area (the allocation-free entry point) and rows wider than it.
 hipError_t launch_qmm(int qt, const uint8_t* packed, const void* x, int xdt, void* y, int ydt, int64_t M, int64_t N,
                       int K, const DevTables& tb, int num_cus, const QmmWorkspace& ws, hipStream_t s) {
-  const bool direct = xdt == 1 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
   const int64_t cap = ws.xs ? ws.xs_bytes / (2ll * K) : 0;  // rows the staging area holds
-  if (direct || cap < 1) return launch_qmm_type(qt, packed, x, xdt, y, ydt, M, N, K, tb, num_cus, ws, s);
+  if (qmm_reads_x(x, xdt) || cap < 1) return launch_qmm_type(qt, packed, x, xdt, y, ydt, M, N, K, tb, num_cus, ws, s);
   // pieces of equal height, in whole 256-row tiles where they fit
   const int64_t pieces = (M + cap - 1) / cap;
   int64_t step = (M + pieces - 1) / pieces;

@@ -26,6 +26,7 @@ EXPORTS = {
     "gsq_block_bytes": (_I32, [_I32]),
     "gsq_set_tables": (_I32, [_I32, _VP, _I64, _I64, _VP, _I64]),
     "gsq_prepare": (_I32, [_VP]),
+    "gsq_prepare_staging": (_I32, [_VP]),
     "gsq_tables_ready": (_I32, [_I32]),
     "gsq_dequant": (_I32, [_I32, _VP, _I64, _VP, _VP]),
     "gsq_qmv": (_I32, [_I32, _VP, _VP, _I32, _VP, _I32, _I64, _I64, _I64, _VP]),
@@ -120,11 +121,14 @@ def launch(name: str, device: torch.device, args: tuple, what: str) -> None:
         check(rc, what)
 
 
-def prepare(device=None, stream=None) -> None:
+def prepare(device=None, stream=None, staging: bool = False) -> None:
     """Build the fixed tables and the QMM workspace of ``stream`` (default: the current
     stream) on ``device`` so that later calls on that stream allocate nothing; required
-    before capturing QMM calls on a stream into a HIP graph (``gsq_prepare``)."""
+    before capturing QMM calls on a stream into a HIP graph (``gsq_prepare``). ``staging``: also
+    the area in which fp32, bf16 and unaligned activations are laid out (``gsq_prepare_staging``),
+    which otherwise the first such call outside capture allocates."""
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     with torch.cuda.device(device):
         s = torch.cuda.current_stream(device) if stream is None else stream
-        check(lib().gsq_prepare(s.cuda_stream), "gsq_prepare")
+        name = "gsq_prepare_staging" if staging else "gsq_prepare"
+        check(getattr(lib(), name)(s.cuda_stream), name)

@@ -47,3 +47,36 @@ def test_rows_beyond_the_staging_area():
     h = x.half()
     want = torch.cat([_call("Q4_K", packed, h[a:b], b - a, n, k, 1) for a, b in ((0, 2048), (2048, 4000))])
     assert torch.isfinite(got).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m", [20, 130])
+def test_captured_on_a_prepared_stream(m):
+    """bf16 rows captured on a stream prepared with a staging area: every replay, between eager calls on
+    that stream with other rows, gives the eager result of the aligned fp16 rows."""
+    from mlx_gsq_amd import _lib
+    from mlx_gsq_amd.formats import TYPE_IDS
+    n, k = 520, 1024
+    packed = torch.from_numpy(synth.make_packed("Q4_K", n, k, seed=4)).cuda()
+    x = torch.empty(m, k, dtype=torch.bfloat16, device="cuda")
+    y = torch.empty(m, n, device="cuda")
+    other = torch.randn(m + 30, k, device="cuda")
+    cap = torch.cuda.Stream()
+    _lib.prepare(stream=cap, staging=True)
+    cap.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        rc = _lib.lib().gsq_qmm(TYPE_IDS["Q4_K"], packed.data_ptr(), x.data_ptr(), 2, y.data_ptr(), 0, m, n, k,
+                                cap.cuda_stream)
+    assert rc == 0, _lib.lib().gsq_last_error()
+    torch.cuda.synchronize()
+    for rep in range(3):
+        x.copy_(torch.randn(m, k, generator=torch.Generator().manual_seed(rep)))
+        y.fill_(float("nan"))
+        want = _call("Q4_K", packed, x.half(), m, n, k, 1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), f"replay {rep}"
+        with torch.cuda.stream(cap):
+            _call("Q4_K", packed, other, m + 30, n, k, 0)
+        torch.cuda.synchronize()

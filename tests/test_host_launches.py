@@ -84,3 +84,37 @@ for group in ({0, 1, 2, 3}, {4, 5}):  # the workspace's users; the scratch's
         assert seq[i:i + n] == [seq[i]] * n, f"call of thread {seq[i]} interrupted: {seq[i:i + n]}"
         i += n
 """)
+
+
+def test_staging_area_is_made_when_needed(stub):
+    """The 128 MB in which fp32, bf16 and unaligned activations are laid out: not for callers of aligned
+    fp16 rows, asked for again after a failure, never under capture, and by gsq_prepare_staging."""
+    run(stub, """
+MB = 1 << 20
+lib.gsq_prepare_staging.argtypes = [P]
+def big():
+    return [b // MB for b in map(stub.stub_malloc_bytes, range(stub.stub_mallocs())) if b >= MB]
+lib.gsq_prepare(S)
+call(lib.gsq_qmm)
+call(lib.gsq_qmv, x=X + 2, m=1)  # its copy uses the partials' memory
+assert big() == [128], big()  # the partial tiles
+# no room: the generic kernel; the next call asks again
+knob("stub_malloc_limit", MB, ctypes.c_size_t)
+assert counted(lib.gsq_qmm, xdt=BF16) == 1
+knob("stub_malloc_limit", 1 << 40, ctypes.c_size_t)
+assert counted(lib.gsq_qmm, xdt=BF16) == 3
+assert big() == [128, 128]
+assert counted(lib.gsq_qmm, xdt=F32, m=20) == 2 and big() == [128, 128]
+# a stream that captures: nothing is allocated; prepared for it, the staged kernels are captured
+T, U = S + 1, S + 2
+assert lib.gsq_prepare(T) == 0 and lib.gsq_prepare_staging(U) == 0
+assert big() == [128] * 5
+knob("stub_capturing", 1)
+assert counted(lib.gsq_qmm, xdt=BF16, stream=T) == 1
+assert counted(lib.gsq_qmm, xdt=BF16, stream=U) == 3
+assert lib.gsq_prepare_staging(T) != 0 and b"before the stream starts capturing" in lib.gsq_last_error()
+assert big() == [128] * 5
+knob("stub_capturing", 0)
+knob("stub_malloc_limit", MB, ctypes.c_size_t)
+assert lib.gsq_prepare_staging(T) != 0 and b"staging" in lib.gsq_last_error()
+""")
