@@ -373,9 +373,8 @@ static hipError_t launch_attn_seq_t(const AttnSeqArgs& a, hipStream_t s) {
   auto launch = [&](auto hd) -> hipError_t {
     constexpr int HD = decltype(hd)::value;
     constexpr int lds = 2 * 2 * 64 * HD * 2;  // two groups' K and V tiles: 64 rows of 2 hd bytes each
-    static const hipError_t attr = hipFuncSetAttribute((const void*)attn_seq_kernel<BF, HD>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (attr != hipSuccess) return attr;
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise((const void*)attn_seq_kernel<BF, HD>, lds); e != hipSuccess) return e;
     hipLaunchKernelGGL((attn_prep_seq_kernel<BF, HD>), pgrid, dim3(256), 0, s, a);
     hipLaunchKernelGGL((attn_seq_kernel<BF, HD>), grid, dim3(512), lds, s, a);
     return hipGetLastError();

@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace gsq {
 
 enum QType : int {
@@ -179,6 +181,26 @@ struct AttnSeqArgs {
   int64_t qg_stride, k_stride, v_stride, out_stride;
   int B, S, H, Hkv, hd, rd, L;
   float eps;
+};
+
+// A kernel's raised dynamic LDS limit (one static object per kernel): a function attribute belongs to
+// one device, so it is set on each device's first launch, and again after a failure. Devices past
+// the first 64 are not remembered.
+class LdsLimit {
+ public:
+  hipError_t raise(const void* kernel, int bytes) {
+    int dev;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = dev < 64 ? 1ull << dev : 0;
+    if (done_.load(std::memory_order_relaxed) & bit) return hipSuccess;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess) done_.fetch_or(bit, std::memory_order_relaxed);
+    return e;
+  }
+
+ private:
+  std::atomic<uint64_t> done_{0};
 };
 
 // QMM workspace: fp32 partial tiles of workgroups that share an output tile (2 slots per

@@ -1113,14 +1113,8 @@ constexpr int kAttnMaxPositions = 32768;  // scores of up to this many positions
 
 template <int DT>
 static hipError_t attn_lds_attr() {
-  static bool done = false;
-  if (!done) {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_decode_kernel<DT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       kAttnMaxPositions * (int)sizeof(float));
-    if (e != hipSuccess) return e;
-    done = true;
-  }
-  return hipSuccess;
+  static LdsLimit limit;
+  return limit.raise((const void*)attn_decode_kernel<DT>, kAttnMaxPositions * (int)sizeof(float));
 }
 
 hipError_t launch_attn_decode(int dt, const AttnArgs& a, hipStream_t s) {

@@ -813,12 +813,8 @@ static hipError_t launch_mfma_k(const QmmMfmaArgs& a, hipStream_t s) {
   using Plan = QmmPlan<T, MF, WV>;
   static_assert(Plan::kValid);
   auto k = qmm_mfma_kernel<T, MF, MC, A4, WV>;
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, kQLds - Plan::kTbl);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsLimit limit;
+  if (hipError_t e = limit.raise((const void*)k, kQLds - Plan::kTbl); e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3(a.G), dim3(64 * WV), Plan::kLds - Plan::kTbl, s, a);
   return hipGetLastError();
 }

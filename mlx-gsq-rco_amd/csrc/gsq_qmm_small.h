@@ -353,13 +353,8 @@ static hipError_t launch_qms_t(QmsArgs a, hipStream_t s) {
     a.slot_floats = MB * NB * 64 * WV * 4;  // every lane stores MB * NB float4 accumulators
     if (2ll * a.G * a.slot_floats * 4 > a.part_bytes) return hipErrorInvalidValue;
     auto k = qms_kernel<T, A4, WV, NB, HX, MB>;
-    static bool attr_set = false;
-    if (!attr_set) {
-      hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         kQLds - QmsPlan<T, WV, NB, MB>::kTbl);
-      if (e != hipSuccess) return e;
-      attr_set = true;
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise((const void*)k, kQLds - QmsPlan<T, WV, NB, MB>::kTbl); e != hipSuccess) return e;
     constexpr size_t lds = QmsPlan<T, WV, NB, MB>::kLds - QmsPlan<T, WV, NB, MB>::kTbl;
     hipLaunchKernelGGL(k, dim3(a.G), dim3(64 * WV), lds, s, a);
     return hipGetLastError();

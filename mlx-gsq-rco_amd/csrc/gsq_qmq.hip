@@ -305,13 +305,8 @@ static hipError_t launch_qmq_t(const QmvArgs& a, int grid, int threads, size_t l
     return hipFuncGetAttributes(&fa, (const void*)k) != hipSuccess || fa.localSizeBytes > 0;
   }();
   if (spills) return hipErrorNotSupported;
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       160 * 1024 - Qmv<T>::kLds);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsLimit limit;
+  if (hipError_t e = limit.raise((const void*)k, 160 * 1024 - Qmv<T>::kLds); e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3(grid), dim3(threads), lds, s, a);
   return hipGetLastError();
 }

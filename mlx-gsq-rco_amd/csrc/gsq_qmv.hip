@@ -469,24 +469,21 @@ __global__ void __launch_bounds__(qmv_max_threads(qmv_weight(MR, GL, XS))) qmv_k
 template <int T, int MR, bool XS, int GL, int AL, bool PR = false, bool PRE = false>
 static hipError_t launch_qmv_t(const QmvArgs& a, int grid, int threads, size_t lds, hipStream_t s) {
   auto k = qmv_kernel<T, MR, XS, GL, AL, PR, PRE>;
-  // 0: not set up; 1: ready; 2: an AL = 1 build that spills registers (its item-invariant lane
-  // offsets stay live across the loop), replaced by the AL = 0 build of the same variant
-  static int state = 0;
-  if (!state) {
-    hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       160 * 1024 - Qmv<T>::kLds);
-    if (e != hipSuccess) return e;
-    state = 1;
-    if constexpr (AL == 1) {
-      hipFuncAttributes fa;
-      e = hipFuncGetAttributes(&fa, (const void*)k);
-      if (e != hipSuccess) return e;
-      if (fa.localSizeBytes > 0) state = 2;
-    }
-  }
   if constexpr (AL == 1) {
-    if (state == 2) return launch_qmv_t<T, MR, XS, GL, 0, PR, PRE>(a, grid, threads, lds, s);
+    // 0: not asked yet; 2: an AL = 1 build that spills registers (its item-invariant lane offsets
+    // stay live across the loop), replaced by the AL = 0 build of the same variant; 1: one that does not
+    static std::atomic<int> state{0};
+    int st = state.load(std::memory_order_relaxed);
+    if (!st) {
+      hipFuncAttributes fa;
+      hipError_t e = hipFuncGetAttributes(&fa, (const void*)k);
+      if (e != hipSuccess) return e;
+      state.store(st = fa.localSizeBytes > 0 ? 2 : 1, std::memory_order_relaxed);
+    }
+    if (st == 2) return launch_qmv_t<T, MR, XS, GL, 0, PR, PRE>(a, grid, threads, lds, s);
   }
+  static LdsLimit limit;
+  if (hipError_t e = limit.raise((const void*)k, 160 * 1024 - Qmv<T>::kLds); e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3(grid), dim3(threads), lds, s, a);
   return hipGetLastError();
 }
@@ -898,13 +895,8 @@ hipError_t launch_qmv_group2(int qt0, const uint8_t* p0, int64_t N0, void* y0, c
       launch_qmv_rows(qt1, p1, x, DT_F16, y1, ydt, 1, 1, N1, K, tb1, num_cus - c0, s, QmvPre(), &q1) != hipSuccess)
     return hipErrorNotSupported;
   if (q0.gl != 3 || q1.gl != 3 || !q0.a.pair || !q1.a.pair || q0.threads != q1.threads) return hipErrorNotSupported;
-  hipError_t e;
-  static bool attr_set = false;
-  if (!attr_set) {
-    e = hipFuncSetAttribute((const void*)qmv_group_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsLimit limit;
+  if (hipError_t e = limit.raise((const void*)qmv_group_kernel, kLdsBytes); e != hipSuccess) return e;
   const size_t lds = q0.lds > q1.lds ? q0.lds : q1.lds;
   hipLaunchKernelGGL(qmv_group_kernel, dim3(q0.grid + q1.grid), dim3(q0.threads), lds, s, q0.a, q1.a, q0.grid);
   return hipGetLastError();

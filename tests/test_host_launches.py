@@ -118,3 +118,42 @@ knob("stub_capturing", 0)
 knob("stub_malloc_limit", MB, ctypes.c_size_t)
 assert lib.gsq_prepare_staging(T) != 0 and b"staging" in lib.gsq_last_error()
 """)
+
+
+def test_launch_attributes_per_device(stub):
+    """A kernel's dynamic LDS limit is raised on every device it is launched on, and asked for again
+    after a failure."""
+    run(stub, """
+lib.gsq_attn_seq.argtypes = [P, I, P, I, P, I, P, P, P, P, P, P, P, I, P, I, I, I, I, I, I, I, F, ctypes.c_int, P]
+lib.gsq_attn_decode.argtypes = [P, I, P, I, P, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, P, I, ctypes.c_int, P]
+lib.gsq_qmv_group2.argtypes = [ctypes.c_int, P, I, P, ctypes.c_int, P, I, P, P, ctypes.c_int, I, P]
+
+def attn_seq(S_):
+    return lib.gsq_attn_seq(X, 1024, X, 128, X, 128, X, X, X, X, X, X, Y, 512, X, 1, 64, 4, 1, 128, 64, 128, 1e-6, F16, S_)
+
+def attn_decode(S_):
+    return lib.gsq_attn_decode(X, 1024, X, 128, X, 128, X, X, X, X, X, X, Y, 512, 1, 4, 1, 128, 64, 128, 1e-6, None, 0, F16, S_)
+
+def product(fn, m):
+    return lambda S_: fn(Q4_K, PACKED, X, F16, Y, F32, m, 17408, 5120, S_)
+
+def group(S_):
+    return lib.gsq_qmv_group2(Q4_K, PACKED, 17408, Y, Q4_K, PACKED, 17408, Y + (1 << 20), X, F32, 5120, S_)
+
+# prompt and single-token attention; the vector, quad-row and shared matrix-vector kernels; the
+# small-batch and the tiled product
+for i, fn in enumerate((attn_seq, attn_decode, product(lib.gsq_qmv, 1), product(lib.gsq_qmv, 4), group,
+                        product(lib.gsq_qmm, 40), product(lib.gsq_qmm, 512))):
+    knob("stub_device", 0)
+    lib.gsq_prepare(S + i)
+    stub.stub_clear()
+    knob("stub_attr_fails", 1)
+    assert fn(S + i) != 0, i
+    assert stub.stub_launches() == 0, i
+    knob("stub_attr_fails", 0)
+    for device in (0, 1, 1, 0, 70, 70):
+        knob("stub_device", device)
+        assert fn(S + i) == 0, (i, lib.gsq_last_error())
+    got = [stub.stub_attr_device(j) for j in range(stub.stub_attrs())]
+    assert got == [0, 1, 70, 70], (i, got)  # past the 64 devices that are remembered: every time
+""")
