@@ -222,7 +222,6 @@ struct QmmMfmaArgs {
   int tbl_bytes;         // multiple of 16
   float* part;           // 2 * G partial slots of slot_floats
   int slot_floats;       // floats per partial slot: MC * NB * 64 * WV * 4 (a tile)
-  long long part_bytes;  // capacity of `part`
 };
 
 // A partial tile goes to the workspace as whole 16-byte stores in accumulator order (block (i, j)
@@ -875,7 +874,6 @@ static hipError_t launch_mfma(QmmMfmaArgs& a, int num_cus, const QmmWorkspace& w
   }
   a.xcd_remap = (a.G % 8 == 0) ? 1 : 0;
   a.part = ws.part;
-  a.part_bytes = ws.part_bytes;
   switch (mc) {
     case 4: return launch_mfma_t<T, 4, 4, 4>(a, a4, s);
     case 8: return launch_mfma_t<T, 8, 8, 8>(a, a4, s);
@@ -888,7 +886,7 @@ static hipError_t launch_mfma(QmmMfmaArgs& a, int num_cus, const QmmWorkspace& w
 // Q6_K and Q2_K, whose fragment decoders share few field reads between a group's octets (at
 // M = 4 and 16 on 17408 / 8192 / 4096-row products: the codebook types 1-17% faster, IQ4_XS
 // 2-8%, Q4_K 1-7%, Q2_K -1 to +3%, Q6_K 8-16% slower). GSQ_QMS_HX=0 / 1 sets it for every type
-// (read once, for measurements).
+// at up to 16 activation rows (read once, for measurements).
 template <int T>
 constexpr bool qms_group_layout() { return T != Q6_K && T != Q2_K; }
 
