@@ -45,6 +45,7 @@ from dataclasses import dataclass
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 
 @dataclass(frozen=True)
@@ -225,6 +226,11 @@ class GatedDeltaNet(torch.nn.Module):
         return self.out_proj(out.to(x.dtype).reshape(B, S, hv * dv))
 
 
+def _has_derivative(t) -> bool:
+    """Whether autograd records what is done with t, in reverse or forward mode."""
+    return (torch.is_grad_enabled() and t.requires_grad) or forward_ad.unpack_dual(t).tangent is not None
+
+
 def _rotate_half(x):
     h = x.shape[-1] // 2
     return torch.cat([-x[..., h:], x[..., :h]], dim=-1)
@@ -263,15 +269,19 @@ class FullAttention(torch.nn.Module):
         """qk_proj of the row its prologue forms from x (``forward_pre`` keywords)."""
         return self.qk_proj.forward_pre(x, "add_rms_norm", **kw)
 
-    def _seq_kernel(self, qk, v, cache) -> bool:
+    def _seq_kernel(self, x, qk, v, cache) -> bool:
         """Whether the prompt kernel takes these tensors: one 16-bit dtype throughout, a head dim it
-        is built for, contiguous rows at its alignments; the torch formulation runs otherwise."""
+        is built for, contiguous rows at its alignments, within its limits, and no derivative to be
+        carried through them; the torch formulation runs otherwise."""
         from ..runtime.kernels.model_ops import ATTN_SEQ_HEAD_DIMS
-        a_ = self.args
-        kc, vc = cache.k[self.layer], cache.v[self.layer]
-        return (qk.dtype in (torch.float16, torch.bfloat16) and a_.head_dim in ATTN_SEQ_HEAD_DIMS
-                and all(t.dtype == qk.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (qk, v, kc, vc))
-                and self.q_norm_w.dtype == self.k_norm_w.dtype == qk.dtype and qk.shape[1] <= kc.shape[2])
+        a_, norms = self.args, (self.q_norm_w, self.k_norm_w)
+        rows = (qk, v, cache.k[self.layer], cache.v[self.layer])
+        return (qk.dtype in (torch.float16, torch.bfloat16) and x.dtype == qk.dtype
+                and a_.head_dim in ATTN_SEQ_HEAD_DIMS
+                and all(t.dtype == qk.dtype and t.is_contiguous() for t in (*rows, *norms))
+                and all(t.data_ptr() % 16 == 0 for t in rows) and self.inv_freq.dtype == torch.float64
+                and qk.shape[0] <= 65535 and qk.shape[1] <= rows[2].shape[2]
+                and not any(_has_derivative(t) for t in (*rows, *norms)))
 
     def forward(self, x, cache: Qwen35Cache, first=None):
         """``first``: ``qk_proj(x)`` when the caller has computed it already."""
@@ -287,7 +297,7 @@ class FullAttention(torch.nn.Module):
                                         cache.pos, heads=H, kv_heads=Hkv, head_dim=hd, rotary_dim=a_.rotary_dim,
                                         eps=a_.rms_norm_eps)
             return self.o_proj(out.view(B, 1, H * hd))
-        if x.is_cuda and self._seq_kernel(qk, v, cache):
+        if x.is_cuda and self._seq_kernel(x, qk, v, cache):
             from ..runtime.kernels import model_ops
             out = model_ops.attn_seq(qk[..., :H * 2 * hd], qk[..., H * 2 * hd:], v, self.q_norm_w, self.k_norm_w,
                                      self.inv_freq, cache.k[self.layer], cache.v[self.layer], cache.pos, heads=H,

@@ -1,6 +1,6 @@
 """Gated attention of a prompt (``attn_seq``) against float64: token counts around the 16-row waves
 and 64-row tiles, contexts before the prompt that shift the diagonal through the key tiles, every
-head dim, both dtypes; and the model layer's routing to it."""
+head dim, both dtypes."""
 import pytest
 import torch
 
