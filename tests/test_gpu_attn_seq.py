@@ -114,3 +114,90 @@ def test_attn_seq_outside_the_cache():
     assert torch.isfinite(run(12, kc.cuda(), vc.cuda())).all()
     with pytest.raises(ValueError):
         run(0, kc.cuda()[:, :, :16].contiguous(), vc.cuda()[:, :, :16].contiguous())
+
+
+def _seq(case, qk, v, qw, kw, freq, kc, vc):
+    from mlx_gsq_amd.runtime.kernels import model_ops
+    B, S, pos, L, H, G, hd, rd, dtype = case
+    n, d = H * 2 * hd, qk.cuda()
+    gk, gv = kc.cuda(), vc.cuda()
+    out = model_ops.attn_seq(d[..., :n], d[..., n:], v.cuda(), qw.cuda(), kw.cuda(), freq.cuda(), gk, gv,
+                             torch.tensor([pos], device="cuda"), heads=H, kv_heads=G, head_dim=hd, rotary_dim=rd, eps=1e-6)
+    return out.cpu(), gk.cpu(), gv.cpu()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("order", ["rising", "falling", "even tiles", "odd tiles"])
+def test_attn_seq_score_spread(order, dtype):
+    """Scores that rise or fall over hundreds of keys, or lie 45 apart between the even and the odd key
+    tiles: the running maximum moves in every tile, or one of the two wave groups holds nothing
+    that matters. q and k are +-2 throughout (their norm rounds to exactly that), so only the fp32
+    softmax and the output's rounding separate the result from float64."""
+    case = (1, 200, 130, 330, 2, 1, 128, 0, dtype)
+    B, S, pos, L, H, G, hd, rd, _ = case
+    qk, v, qw, kw, freq, kc, vc = _inputs(case, 3)
+    key = torch.arange(L)
+    match = {"rising": key * hd // L, "falling": hd - key * hd // L,
+             "even tiles": (key // 64 % 2 == 0) * 64 + 64 - key % 7, "odd tiles": (key // 64 % 2) * 64 + 64 - key % 7}[order]
+    k = torch.where(torch.arange(hd)[None, :] < match[:, None], 1.0, -1.0).to(dtype)  # agrees with q in `match` dims
+    n = H * 2 * hd
+    qg = qk[..., :n].view(B, S, H, 2 * hd)
+    qg[..., :hd] = 1.0
+    qg[..., hd:] = 20.0  # gates of 1
+    qk[..., n:] = k[pos:]
+    qw[:], kw[:] = 2.0, 2.0
+    kc[0, 0, :pos] = 2 * k[:pos]
+    v, vc = (1 + torch.rand(v.shape, generator=torch.Generator().manual_seed(1))).to(dtype), 1 + vc.abs() % 1
+    want, wk, _ = _reference(qk[..., :n], qk[..., n:], v, qw, kw, freq, kc, vc, pos, H, G, hd, rd, 1e-6)
+    got, gk, _ = _seq(case, qk, v, qw, kw, freq, kc, vc)
+    assert torch.equal(gk, wk)
+    # values in [1, 2]: half a step of the dtype there, plus 1e-5: 2^-24 of exponents up to 80, and
+    # sums of 330 terms
+    half = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert float((got.double() - want).abs().max()) <= half + 1e-5
+
+
+def test_attn_seq_not_finite():
+    """A NaN or infinity reaches the outputs it belongs to and no others."""
+    case = (1, 150, 20, 300, 4, 2, 64, 16, torch.float16)
+    B, S, pos, L, H, G, hd, rd, dtype = case
+    qk, v, qw, kw, freq, kc, vc = _inputs(case, 4)
+    n, t = H * 2 * hd, 70
+    clean, ck, cv = _seq(case, qk, v, qw, kw, freq, kc, vc)
+    assert torch.isfinite(clean).all()
+
+    def run(qk=qk, v=v, kc=kc, vc=vc):
+        return _seq(case, qk, v, qw, kw, freq, kc, vc)[0]
+
+    def check(got, bad):
+        assert torch.isnan(got[bad]).all() and torch.equal(got[~bad], clean[~bad])
+    bad = torch.zeros(B, S, H, hd, dtype=torch.bool)
+    x = qk.clone()  # a query: its row and head
+    x[0, t, 1 * 2 * hd + 5] = float("nan")
+    b = bad.clone()
+    b[0, t, 1] = True
+    check(run(qk=x), b.view(B, S, -1))
+    x = qk.clone()  # a gate: its value
+    x[0, t, 2 * 2 * hd + hd + 7] = float("nan")
+    b = bad.clone()
+    b[0, t, 2, 7] = True
+    check(run(qk=x), b.view(B, S, -1))
+    for bad_value in (float("nan"), float("inf")):  # a key: rows from its token on, of its query heads
+        x = qk.clone()
+        x[0, t, n + hd + 9] = bad_value
+        b = bad.clone()
+        b[0, t:, 2:] = True
+        check(run(qk=x), b.view(B, S, -1))
+    # a value: its dim, from its token on (and, masked by a weight of 0, before it in its key tile)
+    y = v.clone()
+    y[0, t, hd + 11] = float("inf")
+    got = run(v=y).view(B, S, H, hd)
+    c = clean.view(B, S, H, hd)
+    assert not torch.isfinite(got[0, t:, 2:, 11]).any()
+    other = torch.ones(H, hd, dtype=torch.bool)
+    other[2:, 11] = False
+    assert torch.equal(got[:, :, other], c[:, :, other])
+    # positions past the new tokens hold anything
+    kc2, vc2 = kc.clone(), vc.clone()
+    kc2[:, :, pos + S:], vc2[:, :, pos + S:] = float("nan"), float("inf")
+    assert torch.equal(run(kc=kc2, vc=vc2), clean)

@@ -72,3 +72,44 @@ def test_gdn_seq_matches_float64(case):
     assert err(got, want) <= half_ulp + 2e-6
     assert err(grec, wrec) <= 2e-6
     assert torch.equal(gconv.cpu().double(), wconv)
+
+
+@pytest.mark.parametrize("dk", [128, 96])  # column-split kernels; the whole-head one
+def test_gdn_seq_not_finite(dk):
+    """A NaN in one token's value reaches that head's outputs from there on and its state's column, and
+    nothing else; a NaN or infinity in a state likewise."""
+    from mlx_gsq_amd.runtime.kernels import model_ops
+    B, S, hk, hv, dv, K = 1, 50, 2, 4, 64, 4
+    g = torch.Generator().manual_seed(dk)
+    C = 2 * hk * dk + hv * dv
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).half()
+    qkv, z, ab, conv, cw, nw = rnd(B, S, C), rnd(B, S, hv * dv), rnd(B, S, 2 * hv), rnd(B, K - 1, C), rnd(C, K), rnd(dv)
+    ssm_a, dt = -torch.rand(hv, generator=g), torch.randn(hv, generator=g)
+    rec = torch.randn(B, hv, dk, dv, generator=g)
+
+    def run(qkv=qkv, rec=rec):
+        gconv, grec = conv.cuda(), rec.cuda()
+        out = model_ops.gdn_seq(qkv.cuda(), z.cuda(), ab.cuda(), gconv, cw.cuda(), ssm_a.cuda(), dt.cuda(), grec, nw.cuda(),
+                                key_heads=hk, value_heads=hv, head_k_dim=dk, head_v_dim=dv, eps=1e-6)
+        return out.cpu().view(S, hv, dv), grec.cpu()
+    out0, rec0 = run()
+    assert torch.isfinite(out0).all() and torch.isfinite(rec0).all()
+    t, h, j = 21, 2, 37
+    x = qkv.clone()
+    x[0, t, 2 * hk * dk + h * dv + j] = float("nan")
+    out, r = run(qkv=x)
+    bad = torch.zeros(S, hv, dtype=torch.bool)
+    bad[t:, h] = True
+    assert torch.isnan(out[bad]).all() and torch.equal(out[~bad], out0[~bad])
+    col = torch.zeros(hv, dv, dtype=torch.bool)
+    col[h, j] = True
+    assert torch.isnan(r[0].transpose(1, 2)[col]).all()
+    assert torch.equal(r[0].transpose(1, 2)[~col], rec0[0].transpose(1, 2)[~col])
+    for bad_value in (float("nan"), float("inf")):
+        y = rec.clone()
+        y[0, h, 3, j] = bad_value
+        out, r = run(rec=y)
+        assert torch.isnan(out[:, h, j]).all() and torch.equal(out[:, [0, 1, 3]], out0[:, [0, 1, 3]])
+        assert torch.equal(r[0].transpose(1, 2)[~col], rec0[0].transpose(1, 2)[~col])

@@ -80,3 +80,34 @@ def test_captured_on_a_prepared_stream(m):
         with torch.cuda.stream(cap):
             _call("Q4_K", packed, other, m + 30, n, k, 0)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("m", [12, 90, 200])  # small-batch kernel, one and six blocks; tiled kernel
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("qtype", ["Q4_K", "IQ2_S"])
+def test_rows_not_finite(qtype, dtype, m):
+    """NaN, infinities and values past fp16's range stay in their rows, where the outputs are those of
+    the kernel that stages nothing (up to the sign of NaN)."""
+    from mlx_gsq_amd import _lib
+    from mlx_gsq_amd.formats import TYPE_IDS
+    tables.set_tables(tables.synthetic_tables(0))
+    _lib.ensure_tables(qtype, torch.device("cuda:0"))
+    _lib.prepare()
+    n, k = 300, 512
+    packed = torch.from_numpy(synth.make_packed(qtype, n, k, seed=5)).cuda()
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(dtype).cuda()
+    clean = _call(qtype, packed, x, m, n, k, _lib.DTYPE_CODES[dtype])
+    rows = [1, 2, m - 1] if dtype == torch.float16 else [1, 2, 5, m - 1]
+    x[1, 300], x[2, 7], x[m - 1, 511] = float("nan"), float("inf"), float("-inf")
+    if dtype != torch.float16:
+        x[5, 100] = 1e5
+    got = _call(qtype, packed, x, m, n, k, _lib.DTYPE_CODES[dtype])
+    ref, xf = torch.full((m, n), 0.5, device="cuda"), x.float()
+    rc = _lib.lib().gsq_qmm_noalloc(TYPE_IDS[qtype], packed.data_ptr(), xf.data_ptr(), 0, ref.data_ptr(), 0, m, n, k,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.lib().gsq_last_error()
+    fine = torch.ones(m, dtype=torch.bool)
+    fine[rows] = False
+    assert torch.isfinite(clean).all() and torch.equal(got[fine.cuda()], clean[fine.cuda()])
+    assert not torch.isfinite(got[rows]).any()
+    torch.testing.assert_close(got[rows], ref[rows], rtol=0, atol=0, equal_nan=True)
