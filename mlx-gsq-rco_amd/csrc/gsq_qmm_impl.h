@@ -392,11 +392,12 @@ struct QmmTblLds<0> {
 };
 
 // Whether a wave's MFMAs are spread over the phases of its decode (see the stage below) or follow
-// it. Spread: 5-9% faster at 512 and 2048 rows of 17408 x 5120 for IQ3_S and IQ3_XXS, 1-7% for the
-// others, except Q6_K and IQ2_S (2048 rows 570 against 541 us and 448 against 434), whose decodes
-// hold more registers and are better scheduled whole.
+// it. Spread against whole, mean of five shapes, 97 to 2048 rows: the IQ1, IQ2 and IQ3 types 2-11%
+// faster (IQ2_S 17408 x 5120 at 2048 rows 433 against 446 us), Q2_K, Q4_K and IQ4_XS 1% slower to
+// 2.5% faster, Q6_K 1.4% slower at 97 rows to 1.6% faster at 2048 (537 against 538 us there): Q6_K,
+// whose decode holds the most registers, stays whole.
 template <int T>
-constexpr bool qmm_spread() { return T != Q6_K && T != IQ2_S; }
+constexpr bool qmm_spread() { return T != Q6_K; }
 
 template <int T, int MF, int MC, bool A4, int WV>
 __global__ void __launch_bounds__(64 * WV, 1) qmm_mfma_kernel(QmmMfmaArgs args) {
