@@ -238,6 +238,16 @@ int gsq_attn_seq(const void* qg, int64_t qg_stride, const void* k, int64_t k_str
                  int64_t heads, int64_t kv_heads, int64_t head_dim, int64_t rotary_dim, int64_t max_len, float eps,
                  int dtype, void* stream);
 
+/* gsq_attn_seq for a few tokens over a long context: with work not NULL the positions are split into
+ * ceil(max_len / chunk) chunks (chunk a multiple of 128, at most 65535 chunks), one workgroup each
+ * per query tile, whose softmax sums meet in work (batch * heads * seq * ceil(max_len / chunk) *
+ * (head_dim + 2) floats, 16-byte aligned) and are combined by another kernel. */
+int gsq_attn_seq_split(const void* qg, int64_t qg_stride, const void* k, int64_t k_stride, const void* v,
+                       int64_t v_stride, const void* q_norm_w, const void* k_norm_w, const double* inv_freq,
+                       void* k_cache, void* v_cache, const int64_t* pos, void* out, int64_t out_stride, void* q_work,
+                       float* work, int64_t chunk, int64_t batch, int64_t seq, int64_t heads, int64_t kv_heads,
+                       int64_t head_dim, int64_t rotary_dim, int64_t max_len, float eps, int dtype, void* stream);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char* gsq_last_error(void);
 

@@ -4,7 +4,8 @@
 // mlx_gsq/models/qwen35.py:114-152), in two launches:
 //
 //  * attn_prep_seq_kernel: q and k RMS-normalized per head and rotated, k and v into the caches;
-//  * attn_seq_kernel: online-softmax attention over the caches and the sigmoid gate.
+//  * attn_seq_kernel: online-softmax attention over the caches and the sigmoid gate; for a few tokens
+//    over a long context in chunks of positions, whose sums attn_merge_seq_kernel puts together.
 //
 // Before, the torch formulation took tens of launches, float32 copies of the caches, two float32
 // GEMMs over all max_len positions and several passes over a (heads, tokens, max_len) float32
@@ -192,7 +193,12 @@ __global__ void __launch_bounds__(256) attn_prep_seq_kernel(AttnSeqArgs a) {
 //
 // Bound by LDS reads (every wave reads the whole K and V tile: ~2000 cycles a tile of 64 x 64
 // against ~1500 of MFMA); late tiles of the triangle are started first.
-template <bool BF, int HD>
+//
+// SPLIT: workgroup z of a query tile takes positions z * chunk .. + chunk - 1 and leaves its maximum,
+// sum and unnormalized outputs to attn_merge_seq_kernel. A tile's chain of key tiles costs 29 ns a
+// position, and 2 tokens of 24 heads are 24 workgroups: unsplit 956 us over 32768 positions and 4070
+// over 131072 (the torch formulation 722 and 1748), in 8 and 10 chunks 189 and 550.
+template <bool BF, int HD, bool SPLIT>
 __global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
   using E = A16<BF>;
   constexpr int NO = HD / 8, KS = HD / 32, NI = NO / 4, DB = HD / 16, RB = HD * 2;  // RB: bytes of a row
@@ -209,12 +215,17 @@ __global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
   const bool on = tw + c < a.S;
   uint16_t* const out = static_cast<uint16_t*>(a.out) + ((int64_t)bb * a.S + t) * a.out_stride + (int64_t)h * HD;
   if (seq_pos_invalid(a)) {
-    if (on && grp == 0)
+    if (!SPLIT && on && grp == 0)
       for (int i = 0; i < DB; ++i)
         for (int e = 0; e < 4; ++e) out[16 * i + 4 * g + e] = E::mk(__builtin_nanf(""));
     return;
   }
   const int pos = (int)a.pos[0], len = pos + a.S;
+  // key tiles kt_begin .. kt_end - 1, an even number of them unless they end the tile's keys
+  const int nk = (pos + min(t0 + 63, a.S - 1)) / 64 + 1;
+  const int kt_begin = SPLIT ? (int)blockIdx.z * (a.chunk / 64) : 0;
+  const int kt_end = SPLIT ? min(nk, kt_begin + a.chunk / 64) : nk;
+  if (SPLIT && kt_begin >= nk) return;  // every position of the chunk is past the tile's last token
   const int64_t base = ((int64_t)bb * a.Hkv + h / (a.H / a.Hkv)) * a.L * HD;
   const uint16_t* const Kg = static_cast<const uint16_t*>(a.kc) + base;
   const uint16_t* const Vg = static_cast<const uint16_t*>(a.vc) + base;
@@ -228,8 +239,8 @@ __global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
                                        (lds_ptr_t)(dst + (wave * NI + i) * 1024), 16, 0, 0);
     }
   };
-  issue(Kg, kt, 64 * grp, ksw);
-  issue(Vg, vt, 64 * grp, vsw);
+  issue(Kg, kt, 64 * (kt_begin + grp), ksw);
+  issue(Vg, vt, 64 * (kt_begin + grp), vsw);
   u32x4 qf[KS];
   {
     const uint16_t* q = static_cast<const uint16_t*>(a.q) + (((int64_t)bb * a.H + h) * a.S + t) * HD + 8 * g;
@@ -244,16 +255,15 @@ __global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
   // maximum is taken off, and the rounding of (maximum x c) is common to a row
   const float c_ = 1.44269504088896340736f / sqrtf((float)HD);
   const int qpos = pos + t, wmin = pos + min(tw, a.S - 1), wmax = pos + min(tw + 15, a.S - 1);
-  const int nk = (pos + min(t0 + 63, a.S - 1)) / 64 + 1;
   // lane bases of the K and V reads (their swizzles depend on the lane only)
   const uint8_t* const kb = kt + c * RB;
   const int kx = ksw(c), vkey = 4 * g + (c >> 2), vx = vsw(vkey);
   const uint8_t* const vb = vt + vkey * RB + (((c & 3) >> 1) << 4) + ((c & 1) << 3);
   // the query fragments (loaded after the tiles' DMA) are in registers before the loop counts loads
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  for (int kt0 = 0; kt0 < nk; kt0 += 2) {
+  for (int kt0 = kt_begin; kt0 < kt_end; kt0 += 2) {
     const int k0 = (kt0 + grp) * 64;
-    const bool live = k0 <= wmax, more = kt0 + 2 < nk;  // a tile past the wave's last position: barriers only
+    const bool live = k0 <= wmax, more = kt0 + 2 < kt_end;  // a tile past the wave's last position: barriers only
     wait_vm<NI>();  // K has landed (V's DMA may be in flight)
     asm volatile("s_barrier" ::: "memory");
     f32x4 s[4];
@@ -350,6 +360,18 @@ __global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
   const float2 o1 = ml[(grp ^ 1) * 256];
   const float mm = fmaxf(m, o1.x), ms = mm == -INFINITY ? 0.f : mm;
   const float s0 = exp2_raw((m - ms) * c_), s1 = exp2_raw((o1.x - ms) * c_);  // a group without keys: 0 of nothing
+  if constexpr (SPLIT) {
+    const int64_t rows = (int64_t)a.B * a.H * a.S * a.nsplit;
+    const int64_t r = (((int64_t)bb * a.H + h) * a.S + t) * a.nsplit + blockIdx.z;
+    float* const po = a.part + r * HD + 16 * grp * HB + 4 * g;
+#pragma unroll
+    for (int i = 0; i < HB; ++i)
+      *reinterpret_cast<f32x4*>(po + 16 * i) =
+          (grp ? acc[HB + i] : acc[i]) * s0 + mo[(grp ^ 1) * 4 * HB * 64 + i * 64] * s1;
+    if (grp == 0 && g == 0)
+      *reinterpret_cast<float2*>(a.part + rows * HD + 2 * r) = make_float2(mm, l * s0 + o1.y * s1);
+    return;
+  }
   const float inv = 1.f / (l * s0 + o1.y * s1);
   const uint16_t* gate = static_cast<const uint16_t*>(a.qg) + ((int64_t)bb * a.S + t) * a.qg_stride + (int64_t)h * 2 * HD + HD;
 #pragma unroll
@@ -366,17 +388,62 @@ __global__ void __launch_bounds__(512, 2) attn_seq_kernel(AttnSeqArgs a) {
   }
 }
 
+// Outputs of a split prompt: a wave per (row, head, token) weighs the chunks that hold positions of the
+// token by their maxima, as the wave groups are merged above, normalizes and gates. Bound by reading
+// the partial outputs once (24 heads, 16 tokens, 10 chunks of 256 dims: 3.9 MB).
+template <bool BF, int HD>
+__global__ void __launch_bounds__(256) attn_merge_seq_kernel(AttnSeqArgs a) {
+  using E = A16<BF>;
+  constexpr int V = HD / 64;
+  const int64_t rows = (int64_t)a.B * a.H * a.S, i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= rows) return;
+  const int d = V * (threadIdx.x & 63), t = (int)(i % a.S), h = (int)(i / a.S % a.H);
+  const int64_t tok = i / a.S / a.H * a.S + t;
+  uint16_t* const out = static_cast<uint16_t*>(a.out) + tok * a.out_stride + (int64_t)h * HD + d;
+  const uint16_t* const gate = static_cast<const uint16_t*>(a.qg) + tok * a.qg_stride + (int64_t)h * 2 * HD + HD + d;
+  const bool invalid = seq_pos_invalid(a);
+  const int nz = invalid ? 0 : (int)((a.pos[0] + t) / a.chunk) + 1;
+  const float* const po = a.part + i * a.nsplit * HD + d;
+  const float2* const ml = reinterpret_cast<const float2*>(a.part + rows * a.nsplit * HD) + i * a.nsplit;
+  const float c_ = 1.44269504088896340736f / sqrtf((float)HD);
+  float m = -INFINITY, l = 0.f, o[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) o[j] = 0.f;
+  for (int z = 0; z < nz; ++z) m = fmaxf(m, ml[z].x);
+  const float ms = m == -INFINITY ? 0.f : m;
+  for (int z = 0; z < nz; ++z) {
+    const float w = exp2_raw((ml[z].x - ms) * c_);
+    l += ml[z].y * w;
+#pragma unroll
+    for (int j = 0; j < V; ++j) o[j] += po[(int64_t)z * HD + j] * w;
+  }
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int j = 0; j < V; ++j)
+    out[j] = E::mk(invalid ? __builtin_nanf("") : o[j] * inv * (1.f / (1.f + expf(-E::ld(gate[j])))));
+}
+
 template <bool BF>
 static hipError_t launch_attn_seq_t(const AttnSeqArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)((a.S + 63) / 64 * a.H), (unsigned)a.B);
+  const dim3 grid((unsigned)((a.S + 63) / 64 * a.H), (unsigned)a.B, (unsigned)a.nsplit);
   const dim3 pgrid((unsigned)a.S, (unsigned)a.B);
   auto launch = [&](auto hd) -> hipError_t {
     constexpr int HD = decltype(hd)::value;
     constexpr int lds = 2 * 2 * 64 * HD * 2;  // two groups' K and V tiles: 64 rows of 2 hd bytes each
-    static LdsLimit limit;
-    if (hipError_t e = limit.raise((const void*)attn_seq_kernel<BF, HD>, lds); e != hipSuccess) return e;
+    const bool split = a.nsplit > 1;
+    const int64_t rows = (int64_t)a.B * a.H * a.S;
+    if (split && (rows + 3) / 4 >= (1ll << 31)) return hipErrorInvalidValue;
+    static LdsLimit limit, split_limit;
+    const hipError_t e = split ? split_limit.raise((const void*)attn_seq_kernel<BF, HD, true>, lds)
+                               : limit.raise((const void*)attn_seq_kernel<BF, HD, false>, lds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((attn_prep_seq_kernel<BF, HD>), pgrid, dim3(256), 0, s, a);
-    hipLaunchKernelGGL((attn_seq_kernel<BF, HD>), grid, dim3(512), lds, s, a);
+    if (split) {
+      hipLaunchKernelGGL((attn_seq_kernel<BF, HD, true>), grid, dim3(512), lds, s, a);
+      hipLaunchKernelGGL((attn_merge_seq_kernel<BF, HD>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, a);
+    } else {
+      hipLaunchKernelGGL((attn_seq_kernel<BF, HD, false>), grid, dim3(512), lds, s, a);
+    }
     return hipGetLastError();
   };
   if (a.hd == 256) return launch(std::integral_constant<int, 256>{});

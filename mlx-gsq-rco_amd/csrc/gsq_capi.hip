@@ -741,6 +741,16 @@ int gsq_attn_seq(const void* qg, int64_t qg_stride, const void* k, int64_t k_str
                  const int64_t* pos, void* out, int64_t out_stride, void* q_work, int64_t batch, int64_t seq,
                  int64_t heads, int64_t kv_heads, int64_t head_dim, int64_t rotary_dim, int64_t max_len, float eps,
                  int dtype, void* stream) {
+  return gsq_attn_seq_split(qg, qg_stride, k, k_stride, v, v_stride, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos,
+                            out, out_stride, q_work, nullptr, 0, batch, seq, heads, kv_heads, head_dim, rotary_dim, max_len,
+                            eps, dtype, stream);
+}
+
+int gsq_attn_seq_split(const void* qg, int64_t qg_stride, const void* k, int64_t k_stride, const void* v,
+                       int64_t v_stride, const void* q_norm_w, const void* k_norm_w, const double* inv_freq,
+                       void* k_cache, void* v_cache, const int64_t* pos, void* out, int64_t out_stride, void* q_work,
+                       float* work, int64_t chunk, int64_t batch, int64_t seq, int64_t heads, int64_t kv_heads,
+                       int64_t head_dim, int64_t rotary_dim, int64_t max_len, float eps, int dtype, void* stream) {
   if (dtype != GSQ_F16 && dtype != GSQ_BF16) return fail(GSQ_E_TYPE, "unsupported dtype code %d", dtype);
   if (batch < 0 || batch > 65535 || seq < 0) return fail(GSQ_E_VALUE, "batch must be 0..65535, seq not negative");
   if (batch == 0 || seq == 0) return GSQ_OK;
@@ -761,6 +771,14 @@ int gsq_attn_seq(const void* qg, int64_t qg_stride, const void* k, int64_t k_str
     return fail(GSQ_E_VALUE, "rows of qg and out must be 8-byte aligned");
   if (!(eps >= 0.f)) return fail(GSQ_E_VALUE, "eps must be >= 0");
   AttnSeqArgs a;
+  if (work) {
+    if (chunk < 128 || chunk % 128 || chunk > (1ll << 31) || (max_len + chunk - 1) / chunk > 65535)
+      return fail(GSQ_E_VALUE, "chunk must be a multiple of 128, for at most 65535 chunks");
+    if (reinterpret_cast<uintptr_t>(work) & 15) return fail(GSQ_E_VALUE, "work must be 16-byte aligned");
+    a.part = work;
+    a.nsplit = (int)((max_len + chunk - 1) / chunk);
+    a.chunk = a.nsplit > 1 ? (int)chunk : 0;
+  }
   a.qg = qg; a.k = k; a.v = v; a.q_norm_w = q_norm_w; a.k_norm_w = k_norm_w; a.inv_freq = inv_freq;
   a.kc = k_cache; a.vc = v_cache; a.pos = pos; a.q = q_work; a.out = out;
   a.qg_stride = qg_stride; a.k_stride = k_stride; a.v_stride = v_stride; a.out_stride = out_stride;

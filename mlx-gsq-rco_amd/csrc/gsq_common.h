@@ -180,6 +180,10 @@ struct AttnSeqArgs {
   int64_t qg_stride, k_stride, v_stride, out_stride;
   int B, S, H, Hkv, hd, rd, L;
   float eps;
+  // positions split over nsplit workgroups of `chunk` (a multiple of 128) each, whose sums meet in part:
+  // [B, H, S, nsplit] rows of hd floats, then as many (maximum, sum) pairs; nsplit 1: unused
+  float* part = nullptr;
+  int chunk = 0, nsplit = 1;
 };
 
 // A kernel's raised dynamic LDS limit (one static object per kernel): a function attribute belongs to

@@ -42,6 +42,8 @@ EXPORTS = {
                                _I64, _I64, _I64, _I64, _F32, _VP, _I64, _I32, _VP]),
     "gsq_attn_seq": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP, _I64, _I64,
                             _I64, _I64, _I64, _I64, _I64, _F32, _I32, _VP]),
+    "gsq_attn_seq_split": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP, _VP,
+                                  _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F32, _I32, _VP]),
     "gsq_gdn_step": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64,
                             _VP, _I64, _I64, _I64, _I64, _I64, _I64, _F32, _I32, _VP]),
     "gsq_gdn_seq": (_I32, [_VP, _I64, _VP, _I64, _VP, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _VP, _I64,

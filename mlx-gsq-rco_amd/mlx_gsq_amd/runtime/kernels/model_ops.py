@@ -188,13 +188,24 @@ def attn_decode(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos, *
 
 
 ATTN_SEQ_HEAD_DIMS = (64, 128, 256)
+# fewest positions of a chunk when a prompt's are split: a workgroup takes 29 ns a position (~120 us),
+# so shorter caches (8191 positions, 265 us, where the torch formulation took 620) stay whole
+ATTN_SEQ_MIN_CHUNK = 4096
+
+
+def attn_seq_chunk(workgroups: int, max_len: int, cus: int) -> int:
+    """Positions per workgroup of ``attn_seq`` on a device of ``cus`` CUs, each of which holds one: as
+    many chunks as fill the CUs, none shorter than ``ATTN_SEQ_MIN_CHUNK``; 0: not split."""
+    n = min(cus // workgroups, max_len // ATTN_SEQ_MIN_CHUNK)
+    return -(-max_len // (128 * n)) * 128 if n > 1 else 0
 
 
 def attn_seq(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos, *, heads: int, kv_heads: int,
-             head_dim: int, rotary_dim: int, eps: float):
+             head_dim: int, rotary_dim: int, eps: float, chunk=None):
     """``attn_decode`` for a prompt: S new tokens of B rows at positions pos .. pos + S - 1; qg
     (B, S, heads * 2 head_dim), k and v (B, S, kv_heads * head_dim) with unit inner stride and the
-    (B, S) rows at one stride each, fp16 or bf16, head_dim 64, 128 or 256. Returns
+    (B, S) rows at one stride each, fp16 or bf16, head_dim 64, 128 or 256. ``chunk``: positions per
+    workgroup (a multiple of 128; 0 = all; default: ``attn_seq_chunk``). Returns
     (B, S, heads * head_dim)."""
     dev = _on_gpu(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos)
     B, S = qg.shape[0], qg.shape[1]
@@ -215,11 +226,20 @@ def attn_seq(qg, k, v, q_norm_w, k_norm_w, inv_freq, k_cache, v_cache, pos, *, h
         if t.dtype != qg.dtype or not t.is_contiguous():
             raise ValueError("norm weights and caches must be contiguous in the activation dtype")
     out = torch.empty(B, S, heads * head_dim, dtype=qg.dtype, device=dev)
-    work = torch.empty(B * heads * S * head_dim, dtype=qg.dtype, device=dev)
+    q_work = torch.empty(B * heads * S * head_dim, dtype=qg.dtype, device=dev)
+    L = k_cache.shape[2]
+    if chunk is None:
+        chunk = 0
+        if L >= 2 * ATTN_SEQ_MIN_CHUNK and B * S:
+            chunk = attn_seq_chunk(B * heads * (-(-S // 64)), L, torch.cuda.get_device_properties(dev).multi_processor_count)
+    work = None
+    if chunk:
+        work = torch.empty(B * heads * S * (-(-L // chunk)) * (head_dim + 2), dtype=torch.float32, device=dev)
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().gsq_attn_seq(
+        _lib.check(_lib.lib().gsq_attn_seq_split(
             qg.data_ptr(), qg.stride(1), k.data_ptr(), k.stride(1), v.data_ptr(), v.stride(1), q_norm_w.data_ptr(),
             k_norm_w.data_ptr(), inv_freq.contiguous().data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-            pos.data_ptr(), out.data_ptr(), out.stride(1), work.data_ptr(), B, S, heads, kv_heads, head_dim,
-            rotary_dim, k_cache.shape[2], float(eps), _dt(qg), _lib.stream_handle(dev)), "attn_seq")
+            pos.data_ptr(), out.data_ptr(), out.stride(1), q_work.data_ptr(), None if work is None else work.data_ptr(),
+            int(chunk), B, S, heads, kv_heads, head_dim, rotary_dim, L, float(eps), _dt(qg), _lib.stream_handle(dev)),
+            "attn_seq")
     return out

@@ -107,6 +107,20 @@ def test_kernel_refuses_derivatives():
         assert not _taken(layer, x, _cache(layer))
 
 
+def test_positions_per_workgroup():
+    """Long caches are split over the CUs that a few query tiles leave idle, into whole pairs of key tiles."""
+    from mlx_gsq_amd.runtime.kernels.model_ops import ATTN_SEQ_MIN_CHUNK, attn_seq_chunk
+    for wgs in (1, 24, 48, 127, 128, 129, 256, 4000):
+        for L in (8192, 8193, 16384, 32768, 100000, 131072, 1 << 20):
+            c = attn_seq_chunk(wgs, L, 256)
+            if wgs > 128:
+                assert c == 0
+                continue
+            n = -(-L // c)
+            assert c % 128 == 0 and c >= ATTN_SEQ_MIN_CHUNK and 1 < n and n * wgs <= 256
+    assert attn_seq_chunk(24, 8191, 256) == 0 and attn_seq_chunk(24, 32768, 256) == 4096
+
+
 def _run(layer, x, cache, device):
     layer, cache, x = copy.deepcopy(layer).to(device), copy.deepcopy(cache), x.to(device)
     cache.pos = cache.pos.to(device)

@@ -116,19 +116,60 @@ def test_attn_seq_outside_the_cache():
         run(0, kc.cuda()[:, :, :16].contiguous(), vc.cuda()[:, :, :16].contiguous())
 
 
-def _seq(case, qk, v, qw, kw, freq, kc, vc):
+def _seq(case, qk, v, qw, kw, freq, kc, vc, chunk=None):
     from mlx_gsq_amd.runtime.kernels import model_ops
     B, S, pos, L, H, G, hd, rd, dtype = case
     n, d = H * 2 * hd, qk.cuda()
     gk, gv = kc.cuda(), vc.cuda()
     out = model_ops.attn_seq(d[..., :n], d[..., n:], v.cuda(), qw.cuda(), kw.cuda(), freq.cuda(), gk, gv,
-                             torch.tensor([pos], device="cuda"), heads=H, kv_heads=G, head_dim=hd, rotary_dim=rd, eps=1e-6)
+                             torch.tensor([pos], device="cuda"), heads=H, kv_heads=G, head_dim=hd, rotary_dim=rd, eps=1e-6,
+                             chunk=chunk)
     return out.cpu(), gk.cpu(), gv.cpu()
 
 
+# (case, positions per workgroup): chunks that start inside, end at and lie past a query tile's last
+# key, a single token of a tile in a chunk, an odd number of key tiles in the last chunk
+SPLITS = [((1, 2, 126, 300, 2, 1, 256, 64, torch.float16), 128), ((2, 3, 255, 1000, 4, 2, 128, 128, torch.float16), 256),
+          ((1, 70, 100, 700, 3, 1, 64, 16, torch.bfloat16), 128), ((1, 16, 1000, 1100, 6, 2, 256, 64, torch.bfloat16), 384),
+          ((1, 130, 0, 900, 2, 1, 128, 32, torch.float16), 128), ((1, 9, 3000, 8192, 24, 4, 256, 64, torch.float16), 1024)]
+
+
+@pytest.mark.parametrize("case,chunk", SPLITS, ids=lambda c: str(c).replace("torch.", ""))
+def test_attn_seq_split(case, chunk):
+    """Positions split over workgroups: the float64 result and the unsplit kernel's, whose sums differ
+    from the split ones in their last fp32 bits only."""
+    B, S, pos, L, H, G, hd, rd, dtype = case
+    t = _inputs(case, 1)
+    want, wk, wv = _reference(t[0][..., :H * 2 * hd], t[0][..., H * 2 * hd:], *t[1:], pos, H, G, hd, rd, 1e-6)
+    got, gk, gv = _seq(case, *t, chunk=chunk)
+    whole, hk, hv = _seq(case, *t, chunk=0)
+
+    def err(a, b):
+        return float((a.double() - b.double()).norm() / b.double().norm())
+    ulp = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    assert torch.equal(gk, hk) and torch.equal(gv, hv)
+    assert err(got, want) <= ulp
+    # a last fp32 bit moves few roundings of the output, one ulp each: a thousandth of the values at most
+    # differ by half an ulp of the largest in 2-norm
+    assert err(got, whole) <= 0.1 * ulp
+
+
+def test_attn_seq_split_outside_the_cache():
+    case = (1, 20, 0, 512, 2, 1, 64, 16, torch.float16)
+    t = _inputs(case, 2)
+    for pos in (493, -1):
+        out, k, v = _seq(case[:2] + (pos,) + case[3:], *t, chunk=128)
+        assert torch.isnan(out).all() and torch.equal(k, t[5]) and torch.equal(v, t[6])
+    assert torch.isfinite(_seq(case[:2] + (492,) + case[3:], *t, chunk=128)[0]).all()
+    for chunk in (64, 200):
+        with pytest.raises(ValueError):
+            _seq(case, *t, chunk=chunk)
+
+
+@pytest.mark.parametrize("chunk", [0, 128])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("order", ["rising", "falling", "even tiles", "odd tiles"])
-def test_attn_seq_score_spread(order, dtype):
+def test_attn_seq_score_spread(order, dtype, chunk):
     """Scores that rise or fall over hundreds of keys, or lie 45 apart between the even and the odd key
     tiles: the running maximum moves in every tile, or one of the two wave groups holds nothing
     that matters. q and k are +-2 throughout (their norm rounds to exactly that), so only the fp32
@@ -149,7 +190,7 @@ def test_attn_seq_score_spread(order, dtype):
     kc[0, 0, :pos] = 2 * k[:pos]
     v, vc = (1 + torch.rand(v.shape, generator=torch.Generator().manual_seed(1))).to(dtype), 1 + vc.abs() % 1
     want, wk, _ = _reference(qk[..., :n], qk[..., n:], v, qw, kw, freq, kc, vc, pos, H, G, hd, rd, 1e-6)
-    got, gk, _ = _seq(case, qk, v, qw, kw, freq, kc, vc)
+    got, gk, _ = _seq(case, qk, v, qw, kw, freq, kc, vc, chunk)
     assert torch.equal(gk, wk)
     # values in [1, 2]: half a step of the dtype there, plus 1e-5: 2^-24 of exponents up to 80, and
     # sums of 330 terms
@@ -157,17 +198,18 @@ def test_attn_seq_score_spread(order, dtype):
     assert float((got.double() - want).abs().max()) <= half + 1e-5
 
 
-def test_attn_seq_not_finite():
+@pytest.mark.parametrize("chunk", [0, 128])
+def test_attn_seq_not_finite(chunk):
     """A NaN or infinity reaches the outputs it belongs to and no others."""
     case = (1, 150, 20, 300, 4, 2, 64, 16, torch.float16)
     B, S, pos, L, H, G, hd, rd, dtype = case
     qk, v, qw, kw, freq, kc, vc = _inputs(case, 4)
     n, t = H * 2 * hd, 70
-    clean, ck, cv = _seq(case, qk, v, qw, kw, freq, kc, vc)
+    clean, _, _ = _seq(case, qk, v, qw, kw, freq, kc, vc, chunk)
     assert torch.isfinite(clean).all()
 
     def run(qk=qk, v=v, kc=kc, vc=vc):
-        return _seq(case, qk, v, qw, kw, freq, kc, vc)[0]
+        return _seq(case, qk, v, qw, kw, freq, kc, vc, chunk)[0]
 
     def check(got, bad):
         assert torch.isnan(got[bad]).all() and torch.equal(got[~bad], clean[~bad])
