@@ -1,11 +1,11 @@
 """gsq_qmm_noalloc (the allocation-free QMM entry point) against gsq_qmm, through the C ABI.
 
 Two calls in a row per kernel, the second with a smaller input, so that the shared scratch
-array holds the first call's partials and counters when the second starts. The small-batch
-kernel (M <= 16) and tiled plans of at most 64 activation rows pick the same launch plan in both
-entry points, so those results are bit-identical; above 64 rows the allocation-free entry point
+array holds the first call's partials and counters when the second starts. Up to 64 activation
+rows (the small-batch kernel, or 64-row tiles) both entry points pick the same launch plan,
+so those results are bit-identical; in the tiled kernel above 64 rows the allocation-free entry point
 uses 64-row tiles (its scratch holds their partials for one workgroup per CU) where gsq_qmm uses
-128- or 256-row tiles, so those results agree within the QMM tolerance (rel-L2 <= 1e-3 and the
+tiles of 128 to 256 rows, so those results agree within the QMM tolerance (rel-L2 <= 1e-3 and the
 reference's rtol 2e-3 / atol 2e-3 * max|ref|, tests/test_all_qmm.py:38-39) and both match the
 oracle to that bar.
 """
